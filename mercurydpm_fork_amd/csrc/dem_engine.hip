@@ -134,9 +134,12 @@ struct Dev {
     uint8_t* rev;
     // the same lists packed back to back per wavefront of 64 particles: the
     // lists of particles 64w .. 64w+63 fill, in order, the region starting at
-    // 64w * stride -- what the force kernel walks.  Each entry holds the list
-    // entry and the reverse slot (0xFF: none) together, one load per entry.
+    // 64w * stride -- what the force kernel walks, gtot[w] entries of it.  Each
+    // entry holds the list entry and what else the kernel needs of it, one
+    // load per entry: reverse slot (0xFF: none) | slot in the owner's own
+    // list << 8 | owner's lane << 14.
     uint2* nbrc;
+    uint32_t* gtot;
     // contact records
     Rec<NS>* rec[2];
     unsigned long long* mask[2];
@@ -334,13 +337,20 @@ __device__ inline bool integrate(const Params& p, bool after, bool before, doubl
     double q[4] = {qq.x, qq.y, qq.z, qq.w};
     const double dt = p.dt;
     bool flag = false;
-    if (after && inv_mass != 0.0) {
-        v = vadd(v, vmul(vmul(vmul(F, inv_mass), 0.5), dt));
+    // the two half-kicks between two drifts add the same increments: neither
+    // the force nor the orientation changes between them
+    V3 dv = zero3(), dw = zero3();
+    if (inv_mass != 0.0) {
+        dv = vmul(vmul(vmul(F, inv_mass), 0.5), dt);
         if (p.rotation) {
             double R[6];
             rotate_inv_inertia(q, om.w, R);
-            w = vadd(w, vmul(vmul(sym_mul(R, T), 0.5), dt));
+            dw = vmul(vmul(sym_mul(R, T), 0.5), dt);
         }
+    }
+    if (after && inv_mass != 0.0) {
+        v = vadd(v, dv);
+        if (p.rotation) w = vadd(w, dw);
     }
     if (before) {
         V3 x = xyz(pr);
@@ -350,13 +360,11 @@ __device__ inline bool integrate(const Params& p, bool after, bool before, doubl
             x = vadd(x, step);
             rotate_quaternion(q, vmul(w, dt));
         } else {
-            v = vadd(v, vmul(vmul(vmul(F, inv_mass), 0.5), dt));
+            v = vadd(v, dv);
             step = vmul(v, dt);
             x = vadd(x, step);
             if (p.rotation) {
-                double R[6];
-                rotate_inv_inertia(q, om.w, R);
-                w = vadd(w, vmul(vmul(sym_mul(R, T), 0.5), dt));
+                w = vadd(w, dw);
                 rotate_quaternion(q, vmul(w, dt));
             }
         }
@@ -950,6 +958,7 @@ __global__ void __launch_bounds__(kBlock) k_rematch(Dev<NS> d, Params p, int cur
             if (lane >= sft) incl += t;
         }
         const size_t off = (size_t)(i - lane) * p.maxn + (size_t)(incl - cnt);
+        if (lane == 63 && i - lane < p.n) d.gtot[i >> 6] = (uint32_t)incl;
         if (!valid) continue;
         const uint32_t idi = d.t_id[i];
         unsigned long long m = 0;
@@ -957,6 +966,7 @@ __global__ void __launch_bounds__(kBlock) k_rematch(Dev<NS> d, Params p, int cur
             const size_t sl = lslot(k, p.maxn, i);
             const uint32_t e = d.nbr[sl];
             const uint32_t j = e & ~kWriterBit;
+            const uint32_t at = (uint32_t)k << 8 | (uint32_t)lane << 14;
             if (e & kWriterBit) {
                 Rec<NS> r;
                 if (hash_find(d, ((uint64_t)idi << 32) | d.t_id[j], r)) {
@@ -964,7 +974,7 @@ __global__ void __launch_bounds__(kBlock) k_rematch(Dev<NS> d, Params p, int cur
                     m |= 1ull << k;
                 }
                 d.rev[sl] = 0xFF;
-                d.nbrc[off + k] = make_uint2(e, 0xFFu);
+                d.nbrc[off + k] = make_uint2(e, at | 0xFFu);
             } else {
                 const int cj = d.ncount[j];
                 int kk = -1;
@@ -975,7 +985,7 @@ __global__ void __launch_bounds__(kBlock) k_rematch(Dev<NS> d, Params p, int cur
                     }
                 if (kk < 0) atomicOr(&d.flags[F_LIST_ASYM], 1);
                 d.rev[sl] = (uint8_t)(kk < 0 ? 0xFF : kk);
-                d.nbrc[off + k] = make_uint2(e, kk < 0 ? 0xFFu : (uint32_t)kk);
+                d.nbrc[off + k] = make_uint2(e, at | (kk < 0 ? 0xFFu : (uint32_t)kk));
             }
         }
         d.mask[cur][i] = m;
@@ -1086,6 +1096,11 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 //            queue order, i.e. in list order: the sum is deterministic.
 // Both particles of a pair evaluate it (no atomics); the lower id writes the
 // history record.
+// A packed list entry names its owner and its slot in the owner's list: finding
+// them by a binary search over the owners' list lengths in LDS cost six
+// dependent LDS reads per entry (2M chute, 600 steps and the state read back:
+// 423 ms with the search and both half-kicks' increments computed apart, 413
+// without).
 
 __device__ inline uint32_t lane_prefix(unsigned long long ballot)
 {
@@ -1119,7 +1134,6 @@ struct OwnerLds {
     double wx[64], wy[64], wz[64], ii[64];
     unsigned long long m_in[64];
     int32_t sp[64];
-    int32_t pre[64];    // exclusive prefix of the owners' list lengths
     int32_t first[64];  // first queue position of each owner in a batch
     unsigned long long q[kQueue];
     double cf[6][64];
@@ -1323,7 +1337,6 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     const int wbase = i - lane;  // the wavefront's particles are wbase .. wbase + 63
     const bool valid = i < p.n;
     const int ii = valid ? i : 0;
-    const int cnt = valid ? d.ncount[ii] : 0;
     {
         // the owners' state goes to LDS for the contact phase; the epilogue
         // reads it back, so that it occupies no registers meanwhile
@@ -1345,17 +1358,9 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
         L.m_in[lane] = valid ? d.mask[cur][ii] : 0ull;
         L.sp[lane] = (int)(d.spc[ii] & 0xFFFF);
     }
-    // the wavefront's lists are walked as one flat sequence of
-    // total = sum(cnt) entries, entry e belonging to the owner o with
-    // pre[o] <= e < pre[o] + cnt[o]
-    int incl = cnt;
-    for (int sft = 1; sft < 64; sft <<= 1) {
-        const int t = __shfl_up(incl, sft, 64);
-        if (lane >= sft) incl += t;
-    }
-    const int total = __shfl(incl, 63, 64);
-    L.pre[lane] = incl - cnt;
-    // the wavefront's packed lists start at wbase * stride
+    // the wavefront's packed lists are walked as one flat sequence of `total`
+    // entries starting at wbase * stride
+    const int total = wbase < p.n ? __builtin_amdgcn_readfirstlane((int)d.gtot[wbase >> 6]) : 0;
     const size_t lbase = (size_t)wbase * p.maxn;
     unsigned long long touched = 0;
     V3 F = zero3(), T = zero3();
@@ -1397,39 +1402,26 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     };
 
     for (int e0 = 0; e0 < total; e0 += 64 * kScanU) {
-        uint32_t ej[kScanU], kr[kScanU];
-        int eo[kScanU], ek[kScanU];
+        uint2 en[kScanU];
         double4 pq[kScanU];
 #pragma unroll
         for (int u = 0; u < kScanU; ++u) {
             const int e = e0 + 64 * u + lane;
-            int o = 0;
-            if (e < total)
-                for (int sft = 32; sft > 0; sft >>= 1)
-                    if (L.pre[o + sft] <= e) o += sft;
-            eo[u] = o;
-            ek[u] = e - L.pre[o];
-            ej[u] = 0u;
-            kr[u] = 0xFFu;
-            if (e < total) {
-                const uint2 nr = d.nbrc[lbase + (size_t)e];
-                ej[u] = nr.x;
-                kr[u] = nr.y;
-            }
+            en[u] = e < total ? d.nbrc[lbase + (size_t)e] : make_uint2(0u, 0u);
         }
 #pragma unroll
         for (int u = 0; u < kScanU; ++u)
-            pq[u] = e0 + 64 * u + lane < total ? d.posr[ej[u] & ~kWriterBit] : make_double4(0.0, 0.0, 0.0, 0.0);
+            pq[u] = e0 + 64 * u + lane < total ? d.posr[en[u].x & ~kWriterBit] : make_double4(0.0, 0.0, 0.0, 0.0);
 #pragma unroll
         for (int u = 0; u < kScanU; ++u) {
             bool contact = false;
             unsigned long long entry = 0;
             if (e0 + 64 * u + lane < total) {
-                const int o = eo[u];
+                const int o = (int)(en[u].y >> 14) & 63;
                 const V3 po = mk(L.px[o], L.py[o], L.pz[o]);
                 const double ro = L.r[o];
-                const uint32_t j = ej[u] & ~kWriterBit;
-                const bool writer = (ej[u] & kWriterBit) != 0;
+                const uint32_t j = en[u].x & ~kWriterBit;
+                const bool writer = (en[u].x & kWriterBit) != 0;
                 V3 xj = xyz(pq[u]);
                 bool img = false, exists = true;
                 int codes = 0;
@@ -1446,19 +1438,15 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
                 }
                 if (!img || exists) {
                     const bool i_is_P = img || writer;
-                    const V3 posP = i_is_P ? po : xj;
-                    const V3 posI = i_is_P ? xj : po;
-                    const double rP = i_is_P ? ro : pq[u].w;
-                    const double rI = i_is_P ? pq[u].w : ro;
-                    const V3 branch = vsub(posP, posI);
-                    const double d2 = vlen2(branch);
-                    const double sum_r = rI + rP;
+                    // (the same squares and the same sum whichever side is P)
+                    const double d2 = vlen2(vsub(po, xj));
+                    const double sum_r = ro + pq[u].w;
                     if (d2 < sum_r * sum_r) {
                         contact = true;
-                        entry = (unsigned long long)j | ((unsigned long long)ek[u] << 32) |
+                        entry = (unsigned long long)j | ((unsigned long long)((en[u].y >> 8) & 63) << 32) |
                                 ((unsigned long long)o << 38) | ((unsigned long long)codes << 44) |
                                 ((unsigned long long)img << 50) | ((unsigned long long)i_is_P << 51) |
-                                ((unsigned long long)writer << 52) | ((unsigned long long)(kr[u] & 0xFF) << 53);
+                                ((unsigned long long)writer << 52) | ((unsigned long long)(en[u].y & 0xFF) << 53);
                     }
                 }
             }
@@ -2626,7 +2614,7 @@ int alloc_particles(dem_ctx* ctx, int64_t n)
     A(d.t_id, n) A(d.t_orig, n) A(d.t_spc, n) A(d.t_cellc, n);
     const size_t slots = (size_t)n * ctx->maxn_cfg;
     const size_t wslots_packed = ((size_t)n + 63) / 64 * 64 * ctx->maxn_cfg;
-    A(d.nbr, slots) A(d.ncount, n) A(d.rev, slots) A(d.nbrc, wslots_packed);
+    A(d.nbr, slots) A(d.ncount, n) A(d.rev, slots) A(d.nbrc, wslots_packed) A(d.gtot, (n + 63) / 64);
     A(d.rec[0], slots) A(d.rec[1], slots) A(d.mask[0], n) A(d.mask[1], n) A(d.fc, slots) A(d.ftc, slots);
     const size_t wslots = (size_t)n * ctx->wall_slots;
     A(d.wrec[0], wslots) A(d.wrec[1], wslots) A(d.wmask[0], n) A(d.wmask[1], n) A(d.fw, wslots) A(d.ftw, wslots);
