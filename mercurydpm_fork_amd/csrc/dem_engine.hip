@@ -50,6 +50,10 @@ constexpr int kMaxLevels = 4;
 constexpr int kMaxSlabs = 64;
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64; // wavefronts per block
+// Skin of the pruned lists, as a fraction of the Verlet skin: a smaller one
+// keeps fewer entries and prunes more often.  2M chute, us per force pass at
+// 0.08, 0.14, 0.2, 0.3, 0.45: 447, 443, 444, 450, 457 (462 without pruning).
+constexpr double kInnerSkin = 0.2;
 constexpr uint64_t kEmptyKey = ~0ull;
 // marks, in its id, a particle that dem_remove_particles deletes in place
 // (particle ids are below 2^31)
@@ -72,7 +76,8 @@ enum Flag {
     F_DONE_BLOCKS = 12, // blocks of the last rebuild kernel that have finished
     F_NONFINITE = 13,   // a particle position is not finite: the run diverged
     F_STEP = 14,        // the step counter of steps replayed from a captured graph
-    F_NUM = 15
+    F_PRUNE_AT = 15,    // number of the force pass that has to prune the lists (step_pass)
+    F_NUM = 16
 };
 
 // Integration fused into the force kernel: none (a force pass only), the
@@ -98,6 +103,11 @@ struct Params {
     double pleft[3], pright[3], pshift[3];
     double dt, drag, g[3];
     double rmax, skin, thr2;
+    // pruned lists: their skin, the displacement since the last pruning that
+    // asks for the next, and the unit of the position stored with it
+    double inner, inner_thr2, ref_unit;
+    uint32_t pass;     // number of the force pass this launch is, or precedes
+    uint32_t pass_off; // the same minus the step counter (steps of a captured graph)
     uint32_t nt;
     uint32_t alive_min; // stored interactions with an older stamp have been erased
     int kick;           // integration fused into the force pass (KICK_*)
@@ -140,6 +150,10 @@ struct Dev {
     // list << 8 | owner's lane << 14.
     uint2* nbrc;
     uint32_t* gtot;
+    // the entries of nbrc that can come into contact before the next pruning,
+    // in the same layout (k_force)
+    uint2* nbri;
+    uint32_t* itot;
     // contact records
     Rec<NS>* rec[2];
     unsigned long long* mask[2];
@@ -308,6 +322,46 @@ __device__ inline bool rebuild_pending(const int* flags)
 __device__ inline uint32_t step_nt(const Params& p) { return p.step_dev ? *p.step_dev : p.nt; }
 __device__ inline uint32_t step_alive_min(const Params& p) { return p.step_dev ? *p.step_dev : p.alive_min; }
 
+// The number of the force pass of this launch (or that follows it): force
+// passes are counted from the upload on.
+__device__ inline uint32_t step_pass(const Params& p) { return p.step_dev ? *p.step_dev + p.pass_off : p.pass; }
+
+// disp.w holds the displacement at the last pruning as three 21-bit integers
+// in units of p.ref_unit (skin / 2^19, so that it reaches two skins; a larger
+// one is cut off, which only prunes more often).
+__device__ inline long long ref_pack(double v, double unit)
+{
+    const double q = rint(v / unit);
+    const int c = !(q >= -1048575.0) ? -1048575 : (q > 1048575.0 ? 1048575 : (int)q);
+    return (long long)(c & 0x1FFFFF);
+}
+__device__ inline double ref_encode(const Params& p, double4 ds)
+{
+    return __longlong_as_double(ref_pack(ds.x, p.ref_unit) | ref_pack(ds.y, p.ref_unit) << 21 |
+                                ref_pack(ds.z, p.ref_unit) << 42);
+}
+__device__ inline double ref_part(long long w, int at, double unit)
+{
+    return (double)((int)((w >> at) << 11) >> 11) * unit;
+}
+// Whether this displacement asks for the lists to be pruned again.
+__device__ inline bool prune_due(const Params& p, double4 ds)
+{
+    const long long w = __double_as_longlong(ds.w);
+    const double dx = ds.x - ref_part(w, 0, p.ref_unit);
+    const double dy = ds.y - ref_part(w, 21, p.ref_unit);
+    const double dz = ds.z - ref_part(w, 42, p.ref_unit);
+    return !(dx * dx + dy * dy + dz * dz <= p.inner_thr2);
+}
+
+// What integrate() asks of the list upkeep.
+enum { NEEDS_REBUILD = 1, NEEDS_PRUNE = 2 };
+__device__ inline void ask_lists(int* flags, int needs, uint32_t pass)
+{
+    if (needs & NEEDS_REBUILD) atomicOr(&flags[F_REBUILD], 1);
+    if (needs & NEEDS_PRUNE) __atomic_store_n(&flags[F_PRUNE_AT], (int)pass, __ATOMIC_RELAXED);
+}
+
 // floor(v) as a cell coordinate, clamped to +-2^29 (NaN: 0), so that cell
 // ranges stay small and loops over them end for any position.
 __device__ inline int floor_to_cell(double v)
@@ -324,11 +378,11 @@ __device__ inline int floor_to_cell(double v)
 //  (before) BaseParticle::integrateBeforeForceComputation (BaseParticle.cc:
 //           718-752; fixed particles: BaseInteractable.cc:538-609), the
 //           periodic wrap of checkInteractionWithBoundaries (DPMBase.cc:3272,
-//           PeriodicBoundary.cc:374-391) and the Verlet-list displacement
-//           test, whose result it returns.
+//           PeriodicBoundary.cc:374-391) and the displacement tests of the
+//           lists, whose result it returns (NEEDS_*).
 // F and T are the particle's total force and torque of the last force pass.
 // ------------------------------------------------------------------------
-__device__ inline bool integrate(const Params& p, bool after, bool before, double4& pr, double4& vl, double4& om,
+__device__ inline int integrate(const Params& p, bool after, bool before, double4& pr, double4& vl, double4& om,
                                  double4& qq, double4& ds, V3 F, V3 T)
 {
     const double inv_mass = vl.w;
@@ -336,7 +390,7 @@ __device__ inline bool integrate(const Params& p, bool after, bool before, doubl
     V3 w = xyz(om);
     double q[4] = {qq.x, qq.y, qq.z, qq.w};
     const double dt = p.dt;
-    bool flag = false;
+    int needs = 0;
     // the two half-kicks between two drifts add the same increments: neither
     // the force nor the orientation changes between them
     V3 dv = zero3(), dw = zero3();
@@ -376,11 +430,12 @@ __device__ inline bool integrate(const Params& p, bool after, bool before, doubl
         ds.y += step.y;
         ds.z += step.z;
         // (a non-finite displacement asks for a rebuild too, which detects it)
-        flag = !(ds.x * ds.x + ds.y * ds.y + ds.z * ds.z <= p.thr2);
+        if (!(ds.x * ds.x + ds.y * ds.y + ds.z * ds.z <= p.thr2)) needs |= NEEDS_REBUILD;
+        if (prune_due(p, ds)) needs |= NEEDS_PRUNE;
     }
     vl = make_double4(v.x, v.y, v.z, inv_mass);
     om = make_double4(w.x, w.y, w.z, om.w);
-    return flag;
+    return needs;
 }
 
 // Stand-alone integration step (the first half-step of a batch of steps, and
@@ -403,7 +458,7 @@ __global__ void __launch_bounds__(kBlock) k_kick_drift(Dev<NS> d, Params p, int 
         pr = d.posr[i];
         ds = d.disp[i];
     }
-    if (integrate(p, after, before, pr, vl, om, qq, ds, F, T)) atomicOr(&d.flags[F_REBUILD], 1);
+    ask_lists(d.flags, integrate(p, after, before, pr, vl, om, qq, ds, F, T), step_pass(p));
     if (before) {
         d.posr[i] = pr;
         d.quat[i] = qq;
@@ -1057,6 +1112,7 @@ __global__ void __launch_bounds__(kBlock) k_orphans(Dev<NS> d, Params p)
             d.flags[F_DONE_BLOCKS] = 0;
             d.flags[F_REBUILD] = 0;
             d.flags[F_REBUILDS] += 1;
+            d.flags[F_PRUNE_AT] = (int)step_pass(p);
             d.flags[F_ORPH_COUNT0 + (par ^ 1)] = 0;
             d.flags[F_ORPH_PARITY] = par;
         }
@@ -1101,6 +1157,31 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 // dependent LDS reads per entry (2M chute, 600 steps and the state read back:
 // 423 ms with the search and both half-kicks' increments computed apart, 413
 // without).
+//
+// Pruned lists.  Of a Verlet list's 7.3 entries per particle on the chute about
+// 2 are in contact; most of the rest cannot come into contact for many steps,
+// but each cost a list entry, a 32-byte gather of the partner's position and a
+// test in every step.  A pass that prunes walks the whole lists and keeps the
+// entries within the sum of the radii plus a smaller skin (Params::inner), in
+// list order; the passes that follow walk those (about 3 per particle), which
+// holds until some particle has moved half the smaller skin: integrate() then
+// asks the next pass to prune (F_PRUNE_AT carries that pass's number, so a pass
+// and the one that asks never race).  Every contact is found, in the same
+// order, so the results are bit-identical.
+//
+// What bounds it (2M chute, 0.2 to 0.9 contacts per particle): the state alone,
+// read and written with the integration, takes 163 us (770 MB, 4.7 TB/s, the
+// rate of a large copy); walking the pruned lists adds about 80 us and the
+// contacts 70 to 190, waiting for gathers.  437 us per pass with pruning and
+// with the sums taken lane to lane (16 KB less LDS per block), 462 before.
+// Four wavefronts per SIMD (128 registers, spilling) took 491, two lanes
+// loading each record together 441.
+
+// v of lane src
+__device__ inline V3 wave_get(V3 v, int src)
+{
+    return mk(__shfl(v.x, src, 64), __shfl(v.y, src, 64), __shfl(v.z, src, 64));
+}
 
 __device__ inline uint32_t lane_prefix(unsigned long long ballot)
 {
@@ -1112,7 +1193,7 @@ __device__ inline uint32_t lane_prefix(unsigned long long ballot)
 // img << 50 | i_is_P << 51 | writer << 52 | slot of the pair in j's list
 // (0xFF: none) << 53
 #ifndef DEM_SCAN_UNROLL
-#define DEM_SCAN_UNROLL 4
+#define DEM_SCAN_UNROLL 3
 #endif
 // Rounds of 64 list entries each lane loads before testing them
 // (memory-level parallelism).
@@ -1131,12 +1212,10 @@ constexpr int kQueue = 64 + 64 * kScanU;
 struct OwnerLds {
     double px[64], py[64], pz[64], r[64];
     double vx[64], vy[64], vz[64], im[64];
-    double wx[64], wy[64], wz[64], ii[64];
-    unsigned long long m_in[64];
+    double wx[64], wy[64], wz[64];
     int32_t sp[64];
     int32_t first[64];  // first queue position of each owner in a batch
     unsigned long long q[kQueue];
-    double cf[6][64];
 };
 
 __device__ inline int q_owner(unsigned long long e) { return (int)((e >> 38) & 63); }
@@ -1169,8 +1248,10 @@ __device__ inline dem_pair_params pair_params(const dem_pair_params* __restrict_
 
 template <int NS, int LAW, int PREC>
 __device__ inline void process_batch(Dev<NS>& d, const Params& p, int cur, OwnerLds& L, const LawLds& T,
-                                     int wbase, int base, int nb, int lane)
+                                     int wbase, int base, int nb, int lane, V3& cF, V3& cT)
 {
+    cF = zero3();
+    cT = zero3();
     if (lane < nb) {
         const unsigned long long e = L.q[base + lane];
         const uint32_t j = (uint32_t)e;
@@ -1193,16 +1274,14 @@ __device__ inline void process_batch(Dev<NS>& d, const Params& p, int cur, Owner
         // one species: every pair is pair 0, and the partner's species need
         // not be read
         const int sj = p.ns == 1 ? 0 : (int)(d.spc[j] & 0xFFFF);
-        const bool had = writer && ((L.m_in[o] >> k) & 1ull);
         Rec<NS> hist;
         bool has_hist = false;
-        if (had) {
-            hist = rin[slot];
-            has_hist = true;
-        } else if (!writer && kk != 0xFF) {
-            const unsigned long long mj = d.mask[cur][j];
-            hist = rin[lslot((int)kk, p.maxn, (int)j)];
-            has_hist = (mj >> kk) & 1ull;
+        if (writer || kk != 0xFF) {
+            const int hk = writer ? k : (int)kk;
+            const int hi = writer ? i : (int)j;
+            const unsigned long long mh = d.mask[cur][hi];
+            hist = rin[lslot(hk, p.maxn, hi)];
+            has_hist = (mh >> hk) & 1ull;
         }
         Body bi;
         bi.pos = mk(L.px[o], L.py[o], L.pz[o]);
@@ -1245,7 +1324,7 @@ __device__ inline void process_batch(Dev<NS>& d, const Params& p, int cur, Owner
             }
         }
         const dem_pair_params sp = pair_params<LAW>(d.sp, T, p.ns * p.ns <= kLdsPairs, L.sp[o] * p.ns + sj);
-        V3 cF, cT = zero3(), ft;
+        V3 ft;
         if constexpr (PREC == DEM_PRECISION_MIXED) {
             ContactM gm;
             pair_contact_mixed(branch, P.radius, I.radius, P.vel, I.vel, P.omega, I.omega, gm);
@@ -1280,12 +1359,6 @@ __device__ inline void process_batch(Dev<NS>& d, const Params& p, int cur, Owner
                 if (p.rotation) cT = vadd(vneg(tc), vcross(vsub(I.pos, g.contact), f));
             }
         }
-        L.cf[0][lane] = cF.x;
-        L.cf[1][lane] = cF.y;
-        L.cf[2][lane] = cF.z;
-        L.cf[3][lane] = cT.x;
-        L.cf[4][lane] = cT.y;
-        L.cf[5][lane] = cT.z;
         if (writer) {
             Rec<NS> r;
             for (int a = 0; a < NS; ++a) r.s[a] = spring[a];
@@ -1296,7 +1369,7 @@ __device__ inline void process_batch(Dev<NS>& d, const Params& p, int cur, Owner
             // time stamp is newer (InteractionHandler.cc:339-350); with equal
             // stamps (the initial force pass and step 0 both stamp 1) the
             // previous record survives unchanged.
-            if (img && had && hist.ts >= r.ts) r = hist;
+            if (img && has_hist && hist.ts >= r.ts) r = hist;
             d.rec[cur ^ 1][slot] = r;
             if (p.store_fc) {
                 d.fc[slot] = make_double4(cF.x, cF.y, cF.z, p.fc_stamp);
@@ -1354,52 +1427,22 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
         L.wx[lane] = om.x;
         L.wy[lane] = om.y;
         L.wz[lane] = om.z;
-        L.ii[lane] = om.w;
-        L.m_in[lane] = valid ? d.mask[cur][ii] : 0ull;
         L.sp[lane] = (int)(d.spc[ii] & 0xFFFF);
     }
     // the wavefront's packed lists are walked as one flat sequence of `total`
-    // entries starting at wbase * stride
-    const int total = wbase < p.n ? __builtin_amdgcn_readfirstlane((int)d.gtot[wbase >> 6]) : 0;
+    // entries starting at wbase * stride: the pruned ones, or all of them in a
+    // pass that prunes
+    const uint32_t pass = step_pass(p);
+    const bool prune = (uint32_t)__atomic_load_n(&d.flags[F_PRUNE_AT], __ATOMIC_RELAXED) == pass;
+    const uint2* __restrict__ list = prune ? d.nbrc : d.nbri;
+    const int total =
+        wbase < p.n ? __builtin_amdgcn_readfirstlane((int)(prune ? d.gtot : d.itot)[wbase >> 6]) : 0;
     const size_t lbase = (size_t)wbase * p.maxn;
+    uint32_t kept = 0;
     unsigned long long touched = 0;
     V3 F = zero3(), T = zero3();
     int qn = 0;
     wave_sync();
-
-    // Process the queued contacts in batches of 64 (or the remainder when
-    // `all`).  The queue is ordered by owner, then by list position, so each
-    // owner adds its contributions in list order: the sum is deterministic.
-    auto drain = [&](bool all) {
-        int head = 0;
-        while (qn - head >= 64 || (all && qn > head)) {
-            const int nb = qn - head < 64 ? qn - head : 64;
-            wave_sync();
-            process_batch<NS, LAW, PREC>(d, p, cur, L, law, wbase, head, nb, lane);
-            L.first[lane] = -1;
-            wave_sync();
-            if (lane < nb) {
-                const int ow = q_owner(L.q[head + lane]);
-                if (lane == 0 || q_owner(L.q[head + lane - 1]) != ow) L.first[ow] = lane;
-            }
-            wave_sync();
-            for (int a = L.first[lane]; a >= 0 && a < nb; ++a) {
-                const unsigned long long qa = L.q[head + a];
-                if (q_owner(qa) != lane) break;
-                F = vadd(F, mk(L.cf[0][a], L.cf[1][a], L.cf[2][a]));
-                T = vadd(T, mk(L.cf[3][a], L.cf[4][a], L.cf[5][a]));
-                if ((qa >> 52) & 1) touched |= 1ull << ((qa >> 32) & 63);
-            }
-            head += nb;
-        }
-        if (head > 0) {
-            // fewer than 64 left, and head >= 64: source and target are disjoint
-            wave_sync();
-            qn -= head;
-            if (lane < qn) L.q[lane] = L.q[head + lane];
-            wave_sync();
-        }
-    };
 
     for (int e0 = 0; e0 < total; e0 += 64 * kScanU) {
         uint2 en[kScanU];
@@ -1407,14 +1450,14 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
 #pragma unroll
         for (int u = 0; u < kScanU; ++u) {
             const int e = e0 + 64 * u + lane;
-            en[u] = e < total ? d.nbrc[lbase + (size_t)e] : make_uint2(0u, 0u);
+            en[u] = e < total ? list[lbase + (size_t)e] : make_uint2(0u, 0u);
         }
 #pragma unroll
         for (int u = 0; u < kScanU; ++u)
             pq[u] = e0 + 64 * u + lane < total ? d.posr[en[u].x & ~kWriterBit] : make_double4(0.0, 0.0, 0.0, 0.0);
 #pragma unroll
         for (int u = 0; u < kScanU; ++u) {
-            bool contact = false;
+            bool contact = false, near = false;
             unsigned long long entry = 0;
             if (e0 + 64 * u + lane < total) {
                 const int o = (int)(en[u].y >> 14) & 63;
@@ -1436,34 +1479,81 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
                         xj = periodic_shift(p, b, xj);
                     }
                 }
-                if (!img || exists) {
+                // (the same squares and the same sum whichever side is P)
+                const double d2 = vlen2(vsub(po, xj));
+                const double sum_r = ro + pq[u].w;
+                if (prune) near = d2 < (sum_r + p.inner) * (sum_r + p.inner);
+                if (exists && d2 < sum_r * sum_r) {
                     const bool i_is_P = img || writer;
-                    // (the same squares and the same sum whichever side is P)
-                    const double d2 = vlen2(vsub(po, xj));
-                    const double sum_r = ro + pq[u].w;
-                    if (d2 < sum_r * sum_r) {
-                        contact = true;
-                        entry = (unsigned long long)j | ((unsigned long long)((en[u].y >> 8) & 63) << 32) |
-                                ((unsigned long long)o << 38) | ((unsigned long long)codes << 44) |
-                                ((unsigned long long)img << 50) | ((unsigned long long)i_is_P << 51) |
-                                ((unsigned long long)writer << 52) | ((unsigned long long)(en[u].y & 0xFF) << 53);
-                    }
+                    contact = true;
+                    entry = (unsigned long long)j | ((unsigned long long)((en[u].y >> 8) & 63) << 32) |
+                            ((unsigned long long)o << 38) | ((unsigned long long)codes << 44) |
+                            ((unsigned long long)img << 50) | ((unsigned long long)i_is_P << 51) |
+                            ((unsigned long long)writer << 52) | ((unsigned long long)(en[u].y & 0xFF) << 53);
                 }
+            }
+            if (prune) {
+                const unsigned long long nb = __ballot(near);
+                if (near) d.nbri[lbase + kept + lane_prefix(nb)] = en[u];
+                kept += (uint32_t)__popcll(nb);
             }
             const unsigned long long ballot = __ballot(contact);
             if (contact) L.q[qn + lane_prefix(ballot)] = entry;
             qn += __popcll(ballot);
         }
-        if (qn >= 64) drain(false);
+        // Process the queued contacts in batches of 64 (the rest too after the
+        // last entries).  The queue is ordered by owner, then by list
+        // position, so each owner adds its contributions in list order: the
+        // sum is deterministic.
+        const bool last = e0 + 64 * kScanU >= total;
+        int head = 0;
+        while (qn - head >= 64 || (last && qn > head)) {
+            const int nb = qn - head < 64 ? qn - head : 64;
+            V3 cF, cT;
+            L.first[lane] = nb;
+            wave_sync();
+            process_batch<NS, LAW, PREC>(d, p, cur, L, law, wbase, head, nb, lane, cF, cT);
+            // owner | list slot << 7 | writer << 13; past the batch: no owner
+            int tag = 64;
+            if (lane < nb) {
+                const unsigned long long qa = L.q[head + lane];
+                tag = q_owner(qa) | (int)((qa >> 32) & 63) << 7 | (int)((qa >> 52) & 1) << 13;
+                if (lane == 0 || q_owner(L.q[head + lane - 1]) != q_owner(qa)) L.first[q_owner(qa)] = lane;
+            }
+            wave_sync();
+            // every owner takes its contributions, in order, out of the lanes
+            // that evaluated them
+            int a = L.first[lane];
+            while (__any(a < nb)) {
+                const int src = a & 63;
+                const int t = __shfl(tag, src, 64);
+                const V3 f = wave_get(cF, src), m = wave_get(cT, src);
+                const bool mine = a < nb && (t & 127) == lane;
+                if (mine) {
+                    F = vadd(F, f);
+                    T = vadd(T, m);
+                    if (t >> 13) touched |= 1ull << ((t >> 7) & 63);
+                }
+                a = mine ? a + 1 : 64;
+            }
+            head += nb;
+        }
+        if (head > 0) {
+            // fewer than 64 left, and head >= 64: source and target are disjoint
+            wave_sync();
+            qn -= head;
+            if (lane < qn) L.q[lane] = L.q[head + lane];
+            wave_sync();
+        }
     }
-    if (qn > 0) drain(true);
+    if (prune && lane == 0 && wbase < p.n) d.itot[wbase >> 6] = kept;
     if (!valid) return;
     wave_sync();
     const double4 pr = make_double4(L.px[lane], L.py[lane], L.pz[lane], L.r[lane]);
     const double4 vl = make_double4(L.vx[lane], L.vy[lane], L.vz[lane], L.im[lane]);
-    const double4 om = make_double4(L.wx[lane], L.wy[lane], L.wz[lane], L.ii[lane]);
+    const double4 om = make_double4(L.wx[lane], L.wy[lane], L.wz[lane], d.omg[i].w);
     const int si = L.sp[lane];
-    const unsigned long long m_in = L.m_in[lane];
+    const unsigned long long m_in = d.mask[cur][i];
     const bool fixed_i = vl.w == 0.0;
     Body bi;
     bi.pos = xyz(pr);
@@ -1558,6 +1648,10 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
         F = vadd(F, vsub(vmul(mk(p.g[0], p.g[1], p.g[2]), mass), vmul(bi.vel, p.drag)));
     }
     if (p.kick != KICK_BOTH) {
+        if (prune) {
+            const double4 ds = d.disp[i];
+            d.disp[i].w = ref_encode(p, ds);
+        }
         d.frc[i] = make_double4(F.x, F.y, F.z, 0.0);
         d.trq[i] = make_double4(T.x, T.y, T.z, 0.0);
     }
@@ -1569,10 +1663,11 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
         if (before) {
             qq = d.quat[i];
             ds = d.disp[i];
+            if (prune) ds.w = ref_encode(p, ds);
         } else if (p.rotation && !fixed_i) {
             qq = d.quat[i];
         }
-        if (integrate(p, true, before, prn, vln, omn, qq, ds, F, T)) atomicOr(&d.flags[F_REBUILD], 1);
+        ask_lists(d.flags, integrate(p, true, before, prn, vln, omn, qq, ds, F, T), pass + 1);
         d.t_posr[i] = prn;
         d.t_vel[i] = vln;
         d.t_omg[i] = omn;
@@ -2185,7 +2280,10 @@ __global__ void __launch_bounds__(kBlock) k_set_kinematics(Dev<NS> d, Params p, 
         ds.y += nx.y - pr.y;
         ds.z += nx.z - pr.z;
         d.disp[i] = ds;
-        if (!(ds.x * ds.x + ds.y * ds.y + ds.z * ds.z <= p.thr2)) atomicOr(&d.flags[F_REBUILD], 1);
+        ask_lists(d.flags,
+                  (ds.x * ds.x + ds.y * ds.y + ds.z * ds.z <= p.thr2 ? 0 : NEEDS_REBUILD) |
+                      (prune_due(p, ds) ? NEEDS_PRUNE : 0),
+                  p.pass);
         d.posr[i] = make_double4(nx.x, nx.y, nx.z, pr.w);
     }
     if (v) d.vel[i] = make_double4(v[3 * o], v[3 * o + 1], v[3 * o + 2], d.vel[i].w);
@@ -2456,6 +2554,7 @@ struct dem_ctx {
     bool in_step = false; // between dem_step_begin and dem_step_end
     bool diverged = false; // a non-finite position was seen; cleared by an upload
     int64_t fc_pass = 0;  // force passes that stored their contact forces
+    uint32_t passes = 0;  // force passes launched
     int cur = 0;
     Params prm{};
     // device buffers
@@ -2615,6 +2714,7 @@ int alloc_particles(dem_ctx* ctx, int64_t n)
     const size_t slots = (size_t)n * ctx->maxn_cfg;
     const size_t wslots_packed = ((size_t)n + 63) / 64 * 64 * ctx->maxn_cfg;
     A(d.nbr, slots) A(d.ncount, n) A(d.rev, slots) A(d.nbrc, wslots_packed) A(d.gtot, (n + 63) / 64);
+    A(d.nbri, wslots_packed) A(d.itot, (n + 63) / 64);
     A(d.rec[0], slots) A(d.rec[1], slots) A(d.mask[0], n) A(d.mask[1], n) A(d.fc, slots) A(d.ftc, slots);
     const size_t wslots = (size_t)n * ctx->wall_slots;
     A(d.wrec[0], wslots) A(d.wrec[1], wslots) A(d.wmask[0], n) A(d.wmask[1], n) A(d.fw, wslots) A(d.ftw, wslots);
@@ -2659,6 +2759,7 @@ void launch_rebuild(dem_ctx* ctx)
     Dev<NS>& d = dev<NS>(ctx);
     hipStream_t s = ctx->stream;
     ctx->hash_pending = false;
+    ctx->prm.pass = ctx->passes + 1;
     const Params& p = ctx->prm;
     // grid-stride kernels: as many blocks as particles need, at most
     // kRebuildBlocks (a launch with no rebuild pending costs about the time
@@ -2682,6 +2783,7 @@ void launch_force(dem_ctx* ctx, int erase, int kick)
     ctx->prm.erase = erase;
     ctx->prm.nt = (uint32_t)ctx->nt;
     ctx->prm.kick = kick;
+    ctx->prm.pass = ++ctx->passes;
     // the last force pass of a call keeps its contact forces for dem_cg_z
     ctx->prm.store_fc = kick != KICK_BOTH;
     if (ctx->prm.store_fc) ctx->prm.fc_stamp = (double)++ctx->fc_pass;
@@ -2715,6 +2817,7 @@ template <int NS>
 void launch_kick(dem_ctx* ctx, int after, int before)
 {
     Dev<NS>& d = dev<NS>(ctx);
+    ctx->prm.pass = ctx->passes + 1;
     hipLaunchKernelGGL(k_kick_drift<NS>, dim3(grid_for(ctx->n)), dim3(kBlock), 0, ctx->stream, d, ctx->prm, after,
                        before);
 }
@@ -2788,6 +2891,8 @@ std::vector<unsigned char> graph_key(dem_ctx* ctx)
     q.store_fc = 0;
     q.fc_stamp = 0.0;
     q.step_dev = nullptr;
+    q.pass = 0;
+    q.pass_off = ctx->passes + 1 - (uint32_t)ctx->nt;
     const Dev<NS>& d = dev<NS>(ctx);
     const int64_t extra[4] = {ctx->n, (int64_t)ctx->nbuckets, ctx->cur, NS};
     std::vector<unsigned char> k(sizeof q + sizeof d + sizeof extra);
@@ -2824,6 +2929,8 @@ hipGraphExec_t step_graph(dem_ctx* ctx)
         return nullptr;
     }
     ctx->prm.step_dev = (const uint32_t*)(ctx->d_flags + F_STEP);
+    ctx->prm.pass_off = ctx->passes + 1 - (uint32_t)ctx->nt;
+    const uint32_t passes = ctx->passes;
     for (int k = 0; k < 2; ++k) {
         ctx->prm.erase = 1;
         launch_rebuild<NS>(ctx);
@@ -2831,6 +2938,7 @@ hipGraphExec_t step_graph(dem_ctx* ctx)
         hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(1), 0, ctx->stream, ctx->d_flags);
     }
     ctx->prm.step_dev = nullptr;
+    ctx->passes = passes;
     const hipError_t ec = hipStreamEndCapture(ctx->stream, &graph);
     hipGraphExec_t exec = nullptr;
     if (ec != hipSuccess || !graph || hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) {
@@ -2860,6 +2968,7 @@ int run_steps(dem_ctx* ctx, int64_t nsteps)
             hipLaunchKernelGGL(k_step_set, dim3(1), dim3(1), 0, ctx->stream, ctx->d_flags, (uint32_t)ctx->nt);
             for (; s + 2 < nsteps; s += 2) {
                 HIPCHK(hipGraphLaunch(g, ctx->stream));
+                ctx->passes += 2;
                 advance_clock(ctx);
                 advance_clock(ctx);
             }
@@ -2956,6 +3065,7 @@ int run_set_kinematics(dem_ctx* ctx, const double* x, const double* v, const dou
                               ctx->stream));
         dst[a] = (const double*)stage[a];
     }
+    ctx->prm.pass = ctx->passes + 1;
     hipLaunchKernelGGL(k_set_kinematics<NS>, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, d, ctx->prm, dst[0],
                        dst[1], dst[2], dst[3]);
     HIPCHK(hipGetLastError());
@@ -3591,6 +3701,9 @@ static int upload_particles(dem_ctx* ctx, int64_t n, int64_t cap, const uint32_t
     p.skin = skin;
     p.sweep = ctx->sweep_cfg;
     p.thr2 = (0.5 * skin) * (0.5 * skin) * 0.999;
+    p.inner = kInnerSkin * skin;
+    p.inner_thr2 = (0.5 * p.inner) * (0.5 * p.inner) * 0.999;
+    p.ref_unit = skin / 524288.0;
     for (int a = 0; a < 3; ++a) p.axis_pb[a] = -1;
     for (int b = 0; b < p.nper; ++b) {
         p.axis_pb[ctx->periodic[b].axis] = b;

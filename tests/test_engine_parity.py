@@ -939,3 +939,35 @@ def test_removal_reorients_periodic_image_interactions_only():
     assert reversed_pairs > 0
     a, b = assert_forces_close(g, o)
     np.testing.assert_array_equal(a["x"], b["x"])
+
+
+@pytest.mark.parametrize("skin", [0.02, 0.3])
+def test_pruned_lists_follow_fast_and_prescribed_motion(skin):
+    """Spheres that cross the pruned lists' skin every few steps (and the
+    Verlet skin now and then), then a prescribed move of a quarter of the
+    Verlet skin, which has to prune again without a rebuild: the contacts of
+    the oracle, which has no lists, in every step."""
+    sc = S.mixture(n=300, seed=91, lx=6.0, ly=6.0, lz=6.0, inflate=1.08, vmax=4.0, laws="hvm",
+                   periodic=(True, True), walls=("bottom", "top"))
+    g, o = make_pair(sc, skin=skin)
+    g.compute_forces()
+    o.compute_forces()
+    for _ in range(12):
+        g.step(3)
+        o.step(3)
+        assert_contacts_close(g, o)
+    rng = np.random.default_rng(1)
+    for e in (g, o):
+        e.step_begin()
+    x = o.download()["x"]
+    move = rng.normal(0.0, 1.0, x.shape)
+    move *= 0.25 * skin / np.linalg.norm(move, axis=1)[:, None]
+    n0 = g.stats().n_rebuilds
+    for e in (g, o):
+        e.set_kinematics(x=x + move)
+        e.step_end()
+    assert_contacts_close(g, o)
+    assert g.stats().n_rebuilds <= n0 + 1
+    g.step(4)
+    o.step(4)
+    assert_contacts_close(g, o)
