@@ -54,6 +54,17 @@ constexpr int kWaves = kBlock / 64; // wavefronts per block
 // keeps fewer entries and prunes more often.  2M chute, us per force pass at
 // 0.08, 0.14, 0.2, 0.3, 0.45: 447, 443, 444, 450, 457 (462 without pruning).
 constexpr double kInnerSkin = 0.2;
+// Particles up to which a wavefront of the force kernel takes 16 and 32
+// particles instead of 64.  A wavefront's pass is a chain of dependent loads
+// and FP64 arithmetic as long as it has batches of 64 contacts to evaluate;
+// with too few wavefronts to hide it (256 CUs hold 3072), shorter chains on
+// more of them are faster, until the idle lanes of the integration cost more.
+// us per force pass with 16 / 32 / 64:
+//   heaps (rolling friction): 500 spheres 21 / 23 / 29, 4000 22 / 28 / 37,
+//   20,000 26 / 29 / 41, 63,000 45 / 38 / 45, 209,000 124 / 96 / 86;
+//   box: 5000 15 / 16 / 20; Hertz-Mindlin chutes: 17,000 16.8 / 17.5 / 23,
+//   34,000 21 / 20 / 24, 69,000 31 / 25 / 27, 137,000 47 / 36 / 33.
+constexpr int64_t kSmallGroup16 = 24576, kSmallGroup32 = 81920;
 constexpr uint64_t kEmptyKey = ~0ull;
 // marks, in its id, a particle that dem_remove_particles deletes in place
 // (particle ids are below 2^31)
@@ -95,6 +106,7 @@ struct Rec {
 struct Params {
     int n, maxn, nwalls, ns, levels, rotation, nper;
     int wstride; // particle-wall slots per particle (the walls a particle may meet at upload, at least 1)
+    int group;   // particles per wavefront of the force kernel (a power of two, at most 64)
     int wgroups; // 1: a particle meets only its species' group of walls (wgrp), 0: every wall
     int sweep;   // Verlet-list build: DEM_SWEEP_PER_PARTICLE or DEM_SWEEP_WAVEFRONT
     int erase;
@@ -142,12 +154,12 @@ struct Dev {
     uint32_t* nbr;
     int32_t* ncount;
     uint8_t* rev;
-    // the same lists packed back to back per wavefront of 64 particles: the
-    // lists of particles 64w .. 64w+63 fill, in order, the region starting at
-    // 64w * stride -- what the force kernel walks, gtot[w] entries of it.  Each
-    // entry holds the list entry and what else the kernel needs of it, one
-    // load per entry: reverse slot (0xFF: none) | slot in the owner's own
-    // list << 8 | owner's lane << 14.
+    // the same lists packed back to back per wavefront of g = Params::group
+    // particles: the lists of particles gw .. gw+g-1 fill, in order, the
+    // region starting at gw * stride -- what the force kernel walks, gtot[w]
+    // entries of it.  Each entry holds the list entry and what else the kernel
+    // needs of it, one load per entry: reverse slot (0xFF: none) | slot in the
+    // owner's own list << 8 | owner's lane << 14.
     uint2* nbrc;
     uint32_t* gtot;
     // the entries of nbrc that can come into contact before the next pruning,
@@ -1007,13 +1019,14 @@ __global__ void __launch_bounds__(kBlock) k_rematch(Dev<NS> d, Params p, int cur
         const int lane = threadIdx.x & 63;
         const bool valid = i < p.n;
         const int cnt = valid ? d.ncount[i] : 0;
+        const int at_group = lane & (p.group - 1);  // the owner's lane
         int incl = cnt;
-        for (int sft = 1; sft < 64; sft <<= 1) {
+        for (int sft = 1; sft < p.group; sft <<= 1) {
             const int t = __shfl_up(incl, sft, 64);
-            if (lane >= sft) incl += t;
+            if (at_group >= sft) incl += t;
         }
-        const size_t off = (size_t)(i - lane) * p.maxn + (size_t)(incl - cnt);
-        if (lane == 63 && i - lane < p.n) d.gtot[i >> 6] = (uint32_t)incl;
+        const size_t off = (size_t)(i - at_group) * p.maxn + (size_t)(incl - cnt);
+        if (at_group == p.group - 1 && i - at_group < p.n) d.gtot[i / p.group] = (uint32_t)incl;
         if (!valid) continue;
         const uint32_t idi = d.t_id[i];
         unsigned long long m = 0;
@@ -1021,7 +1034,7 @@ __global__ void __launch_bounds__(kBlock) k_rematch(Dev<NS> d, Params p, int cur
             const size_t sl = lslot(k, p.maxn, i);
             const uint32_t e = d.nbr[sl];
             const uint32_t j = e & ~kWriterBit;
-            const uint32_t at = (uint32_t)k << 8 | (uint32_t)lane << 14;
+            const uint32_t at = (uint32_t)k << 8 | (uint32_t)at_group << 14;
             if (e & kWriterBit) {
                 Rec<NS> r;
                 if (hash_find(d, ((uint64_t)idi << 32) | d.t_id[j], r)) {
@@ -1406,10 +1419,12 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     }
     const int lane = threadIdx.x & 63;
     OwnerLds& L = lds[threadIdx.x >> 6];
-    const int i = xcd_block() * blockDim.x + threadIdx.x;
-    const int wbase = i - lane;  // the wavefront's particles are wbase .. wbase + 63
-    const bool valid = i < p.n;
-    const int ii = valid ? i : 0;
+    const int wave = xcd_block() * kWaves + (int)(threadIdx.x >> 6);
+    const int wbase = wave * p.group;  // the wavefront's particles are wbase .. wbase + p.group - 1
+    if (wbase >= p.n) return;
+    const int i = wbase + lane;
+    const bool valid = lane < p.group && i < p.n;
+    const int ii = valid ? i : wbase;
     {
         // the owners' state goes to LDS for the contact phase; the epilogue
         // reads it back, so that it occupies no registers meanwhile
@@ -1435,8 +1450,7 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     const uint32_t pass = step_pass(p);
     const bool prune = (uint32_t)__atomic_load_n(&d.flags[F_PRUNE_AT], __ATOMIC_RELAXED) == pass;
     const uint2* __restrict__ list = prune ? d.nbrc : d.nbri;
-    const int total =
-        wbase < p.n ? __builtin_amdgcn_readfirstlane((int)(prune ? d.gtot : d.itot)[wbase >> 6]) : 0;
+    const int total = __builtin_amdgcn_readfirstlane((int)(prune ? d.gtot : d.itot)[wave]);
     const size_t lbase = (size_t)wbase * p.maxn;
     uint32_t kept = 0;
     unsigned long long touched = 0;
@@ -1546,7 +1560,7 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
             wave_sync();
         }
     }
-    if (prune && lane == 0 && wbase < p.n) d.itot[wbase >> 6] = kept;
+    if (prune && lane == 0) d.itot[wave] = kept;
     if (!valid) return;
     wave_sync();
     const double4 pr = make_double4(L.px[lane], L.py[lane], L.pz[lane], L.r[lane]);
@@ -2713,8 +2727,9 @@ int alloc_particles(dem_ctx* ctx, int64_t n)
     A(d.t_id, n) A(d.t_orig, n) A(d.t_spc, n) A(d.t_cellc, n);
     const size_t slots = (size_t)n * ctx->maxn_cfg;
     const size_t wslots_packed = ((size_t)n + 63) / 64 * 64 * ctx->maxn_cfg;
-    A(d.nbr, slots) A(d.ncount, n) A(d.rev, slots) A(d.nbrc, wslots_packed) A(d.gtot, (n + 63) / 64);
-    A(d.nbri, wslots_packed) A(d.itot, (n + 63) / 64);
+    A(d.nbr, slots) A(d.ncount, n) A(d.rev, slots) A(d.nbrc, wslots_packed) A(d.nbri, wslots_packed);
+    const size_t waves = ((size_t)n + ctx->prm.group - 1) / ctx->prm.group;
+    A(d.gtot, waves) A(d.itot, waves);
     A(d.rec[0], slots) A(d.rec[1], slots) A(d.mask[0], n) A(d.mask[1], n) A(d.fc, slots) A(d.ftc, slots);
     const size_t wslots = (size_t)n * ctx->wall_slots;
     A(d.wrec[0], wslots) A(d.wrec[1], wslots) A(d.wmask[0], n) A(d.wmask[1], n) A(d.fw, wslots) A(d.ftw, wslots);
@@ -2787,7 +2802,8 @@ void launch_force(dem_ctx* ctx, int erase, int kick)
     // the last force pass of a call keeps its contact forces for dem_cg_z
     ctx->prm.store_fc = kick != KICK_BOTH;
     if (ctx->prm.store_fc) ctx->prm.fc_stamp = (double)++ctx->fc_pass;
-    const unsigned g = xcd_grid(grid_for(ctx->n));
+    const uint64_t waves = ((uint64_t)ctx->n + ctx->prm.group - 1) / ctx->prm.group;
+    const unsigned g = xcd_grid((unsigned)((waves + kWaves - 1) / kWaves));
     const bool hm = NS == 3 && ctx->all_hertz_mindlin;
     if (ctx->precision == DEM_PRECISION_MIXED) {
         if (hm)
@@ -3700,6 +3716,7 @@ static int upload_particles(dem_ctx* ctx, int64_t n, int64_t cap, const uint32_t
     p.rmax = rmax;
     p.skin = skin;
     p.sweep = ctx->sweep_cfg;
+    p.group = n <= kSmallGroup16 ? 16 : (n <= kSmallGroup32 ? 32 : 64);
     p.thr2 = (0.5 * skin) * (0.5 * skin) * 0.999;
     p.inner = kInnerSkin * skin;
     p.inner_thr2 = (0.5 * p.inner) * (0.5 * p.inner) * 0.999;

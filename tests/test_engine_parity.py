@@ -971,3 +971,38 @@ def test_pruned_lists_follow_fast_and_prescribed_motion(skin):
     g.step(4)
     o.step(4)
     assert_contacts_close(g, o)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 65])
+def test_force_pass_at_the_edges_of_a_wavefronts_particles(n):
+    """Particle counts around the 16 that a wavefront of the force kernel
+    takes in a small system, spheres of every contact law's general path."""
+    sc = S.mixture(n=n, seed=92, lx=3.5, ly=3.5, lz=3.5, inflate=1.1, laws="full", periodic=(True, True),
+                   walls=("bottom",), fixed_frac=0.0)
+    g, o = make_pair(sc)
+    for e in (g, o):
+        e.compute_forces()
+    assert_contacts_equal(g, o)
+    assert_forces_close(g, o)
+    for e in (g, o):
+        e.step(25)
+    assert_contacts_close(g, o)
+    np.testing.assert_allclose(g.download()["x"], o.download()["x"], rtol=0, atol=1e-9)
+
+
+@pytest.mark.parametrize("n", [24576, 24577, 81920, 81921])
+def test_force_pass_where_the_wavefronts_particles_change(n):
+    """The counts at which a wavefront goes from 16 to 32 and to 64
+    particles: the chute's lattice, inflated into contact."""
+    sc = S.chute_hvm(n_flow=n - 24 * 24, seed=5, l=24.4, depth=10.0)
+    assert sc.state.n == n
+    sc.state.radius[:] *= 1.08
+    g, o = make_pair(sc)
+    for e in (g, o):
+        e.compute_forces()
+    # (the largest neighbours on the lattice touch: 1208 pairs at n = 24576)
+    assert assert_contacts_equal(g, o) > 1000
+    assert_forces_close(g, o)
+    for e in (g, o):
+        e.step(3)
+    assert_contacts_close(g, o)
