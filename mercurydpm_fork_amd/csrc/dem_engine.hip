@@ -72,7 +72,7 @@ constexpr uint32_t kRemovedBit = 0x80000000u;
 
 // device flag words
 enum Flag {
-    F_REBUILD = 0,
+    F_REBUILD = 0,      // 0, or rebuild_at() of the first force pass that needs new lists
     F_LIST_OVERFLOW = 1,
     F_HASH_OVERFLOW = 2,
     F_LIST_ASYM = 3,
@@ -128,6 +128,7 @@ struct Params {
     // in steps replayed from a captured graph: the step counter on the device
     // (nt and alive_min both; nullptr: nt and alive_min above)
     const uint32_t* step_dev;
+    uint32_t* rebuild_word; // F_REBUILD for the host, in its memory
     // grid
     double h[kMaxLevels];       // cell size of a non-periodic axis
     double rmaxl[kMaxLevels];   // largest radius on each level
@@ -366,11 +367,28 @@ __device__ inline bool prune_due(const Params& p, double4 ds)
     return !(dx * dx + dy * dy + dz * dz <= p.inner_thr2);
 }
 
-// What integrate() asks of the list upkeep.
-enum { NEEDS_REBUILD = 1, NEEDS_PRUNE = 2 };
-__device__ inline void ask_lists(int* flags, int needs, uint32_t pass)
+// The rebuild flag: the number of the first force pass that must not run on
+// the present lists, doubled, plus one (so that it is never 0).
+__host__ __device__ inline uint32_t rebuild_at(uint32_t pass) { return pass << 1 | 1u; }
+// Whether force pass `pass` has to wait for that rebuild.  A pass and the
+// drift that it ends with, which asks for the next one, never confuse each
+// other.
+__host__ __device__ inline bool waits_for_rebuild(uint32_t flag, uint32_t pass)
 {
-    if (needs & NEEDS_REBUILD) atomicOr(&flags[F_REBUILD], 1);
+    return flag != 0 && (int32_t)(flag - rebuild_at(pass)) <= 0;
+}
+
+// What integrate() asks of the list upkeep, for the force pass `pass`.
+enum { NEEDS_REBUILD = 1, NEEDS_PRUNE = 2 };
+__device__ inline void ask_lists(const Params& p, int* flags, int needs, uint32_t pass)
+{
+    if (needs & NEEDS_REBUILD) {
+        const int at = (int)rebuild_at(pass);
+        if (__atomic_load_n(&flags[F_REBUILD], __ATOMIC_RELAXED) != at) {
+            __atomic_store_n(&flags[F_REBUILD], at, __ATOMIC_RELAXED);
+            __atomic_store_n(p.rebuild_word, (uint32_t)at, __ATOMIC_RELAXED);
+        }
+    }
     if (needs & NEEDS_PRUNE) __atomic_store_n(&flags[F_PRUNE_AT], (int)pass, __ATOMIC_RELAXED);
 }
 
@@ -470,7 +488,7 @@ __global__ void __launch_bounds__(kBlock) k_kick_drift(Dev<NS> d, Params p, int 
         pr = d.posr[i];
         ds = d.disp[i];
     }
-    ask_lists(d.flags, integrate(p, after, before, pr, vl, om, qq, ds, F, T), step_pass(p));
+    ask_lists(p, d.flags, integrate(p, after, before, pr, vl, om, qq, ds, F, T), step_pass(p));
     if (before) {
         d.posr[i] = pr;
         d.quat[i] = qq;
@@ -1400,8 +1418,11 @@ template <int NS, int LAW, int PREC>
 __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Params p, int cur)
 {
     // a diverged state (non-finite position, found by the rebuild) gets no
-    // force pass: its lists were not rebuilt
+    // force pass: its lists were not rebuilt; neither does one that needs new
+    // lists (the host rebuilds them and launches the pass again: run_passes)
     if (__atomic_load_n(&d.flags[F_NONFINITE], __ATOMIC_RELAXED)) return;
+    const uint32_t pass = step_pass(p);
+    if (waits_for_rebuild((uint32_t)__atomic_load_n(&d.flags[F_REBUILD], __ATOMIC_RELAXED), pass)) return;
     __shared__ OwnerLds lds[kWaves];
     __shared__ LawLds law;
     if constexpr (LAW == LAW_HERTZ_MINDLIN) {
@@ -1447,7 +1468,6 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     // the wavefront's packed lists are walked as one flat sequence of `total`
     // entries starting at wbase * stride: the pruned ones, or all of them in a
     // pass that prunes
-    const uint32_t pass = step_pass(p);
     const bool prune = (uint32_t)__atomic_load_n(&d.flags[F_PRUNE_AT], __ATOMIC_RELAXED) == pass;
     const uint2* __restrict__ list = prune ? d.nbrc : d.nbri;
     const int total = __builtin_amdgcn_readfirstlane((int)(prune ? d.gtot : d.itot)[wave]);
@@ -1681,7 +1701,7 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
         } else if (p.rotation && !fixed_i) {
             qq = d.quat[i];
         }
-        ask_lists(d.flags, integrate(p, true, before, prn, vln, omn, qq, ds, F, T), pass + 1);
+        ask_lists(p, d.flags, integrate(p, true, before, prn, vln, omn, qq, ds, F, T), pass + 1);
         d.t_posr[i] = prn;
         d.t_vel[i] = vln;
         d.t_omg[i] = omn;
@@ -2294,7 +2314,7 @@ __global__ void __launch_bounds__(kBlock) k_set_kinematics(Dev<NS> d, Params p, 
         ds.y += nx.y - pr.y;
         ds.z += nx.z - pr.z;
         d.disp[i] = ds;
-        ask_lists(d.flags,
+        ask_lists(p, d.flags,
                   (ds.x * ds.x + ds.y * ds.y + ds.z * ds.z <= p.thr2 ? 0 : NEEDS_REBUILD) |
                       (prune_due(p, ds) ? NEEDS_PRUNE : 0),
                   p.pass);
@@ -2569,6 +2589,14 @@ struct dem_ctx {
     bool diverged = false; // a non-finite position was seen; cleared by an upload
     int64_t fc_pass = 0;  // force passes that stored their contact forces
     uint32_t passes = 0;  // force passes launched
+    // the lists do not fit the particles (upload, append): rebuild before the
+    // next force pass without asking the device
+    bool lists_stale = false;
+    uint32_t* rebuild_word = nullptr; // pinned host memory: see Params::rebuild_word
+    int* h_flags = nullptr;           // pinned host copy of the flag words
+    hipEvent_t batch_done[2] = {nullptr, nullptr};
+    int64_t since_rebuild = 0;        // force passes since the last rebuild of run_passes
+    int batch = 8;                    // force passes launched together by run_passes
     int cur = 0;
     Params prm{};
     // device buffers
@@ -2621,6 +2649,21 @@ int set_err(dem_ctx* c, int code, const std::string& msg)
         if (e_ != hipSuccess)                                                                    \
             return set_err(ctx, DEM_ERR_DEVICE, std::string(#expr ": ") + hipGetErrorString(e_)); \
     } while (0)
+
+// What the host waits on and reads between force passes (run_passes): the
+// rebuild word on a line of its own, then the flag words, pinned.
+int ensure_host_words(dem_ctx* ctx)
+{
+    for (hipEvent_t& e : ctx->batch_done)
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (ctx->rebuild_word) return DEM_OK;
+    void* v = nullptr;
+    HIPCHK(hipHostMalloc(&v, 128 + sizeof(int) * F_NUM, hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset(v, 0, 128 + sizeof(int) * F_NUM);
+    ctx->h_flags = (int*)((char*)v + 128);
+    ctx->rebuild_word = (uint32_t*)v;
+    return DEM_OK;
+}
 
 template <typename T>
 int dalloc(dem_ctx* ctx, T** p, size_t count)
@@ -2774,6 +2817,7 @@ void launch_rebuild(dem_ctx* ctx)
     Dev<NS>& d = dev<NS>(ctx);
     hipStream_t s = ctx->stream;
     ctx->hash_pending = false;
+    ctx->lists_stale = false;
     ctx->prm.pass = ctx->passes + 1;
     const Params& p = ctx->prm;
     // grid-stride kernels: as many blocks as particles need, at most
@@ -2791,12 +2835,23 @@ void launch_rebuild(dem_ctx* ctx)
     hipLaunchKernelGGL(k_orphans<NS>, g, b, 0, s, d, p);
 }
 
+// The integrated state of a force pass goes to the gather buffers: they
+// become the current ones.
 template <int NS>
-void launch_force(dem_ctx* ctx, int erase, int kick)
+void swap_state(dem_ctx* ctx)
+{
+    Dev<NS>& d = dev<NS>(ctx);
+    std::swap(d.posr, d.t_posr);
+    std::swap(d.vel, d.t_vel);
+    std::swap(d.omg, d.t_omg);
+}
+
+template <int NS>
+void launch_force(dem_ctx* ctx, int erase, int kick, uint32_t nt)
 {
     Dev<NS>& d = dev<NS>(ctx);
     ctx->prm.erase = erase;
-    ctx->prm.nt = (uint32_t)ctx->nt;
+    ctx->prm.nt = nt;
     ctx->prm.kick = kick;
     ctx->prm.pass = ++ctx->passes;
     // the last force pass of a call keeps its contact forces for dem_cg_z
@@ -2821,12 +2876,17 @@ void launch_force(dem_ctx* ctx, int erase, int kick)
                                ctx->prm, ctx->cur);
     }
     ctx->cur ^= 1;
-    if (kick != KICK_NONE) {
-        // the integrated state went to the gather buffers: make it current
-        std::swap(d.posr, d.t_posr);
-        std::swap(d.vel, d.t_vel);
-        std::swap(d.omg, d.t_omg);
-    }
+    if (kick != KICK_NONE) swap_state<NS>(ctx);
+}
+
+// Takes back the bookkeeping of the last launched force pass, which did
+// nothing (run_passes).
+template <int NS>
+void unlaunch_force(dem_ctx* ctx, int kick)
+{
+    --ctx->passes;
+    ctx->cur ^= 1;
+    if (kick != KICK_NONE) swap_state<NS>(ctx);
 }
 
 template <int NS>
@@ -2838,11 +2898,21 @@ void launch_kick(dem_ctx* ctx, int after, int before)
                        before);
 }
 
+// The device's flag words as they are once everything launched has run.
+int read_flags(dem_ctx* ctx)
+{
+    int* f = ctx->h_flags;
+    HIPCHK(hipMemcpyAsync(f, ctx->d_flags, sizeof(int) * F_NUM, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    *ctx->rebuild_word = (uint32_t)f[F_REBUILD];
+    return DEM_OK;
+}
+
 int check_flags(dem_ctx* ctx)
 {
-    int f[F_NUM];
-    HIPCHK(hipMemcpyAsync(f, ctx->d_flags, sizeof f, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    const int r = read_flags(ctx);
+    if (r) return r;
+    const int* f = ctx->h_flags;
     ctx->last_rebuilds = ctx->rebuilds_before + f[F_REBUILDS];
     ctx->max_list = f[F_MAX_LIST];
     if (f[F_LIST_OVERFLOW])
@@ -2868,19 +2938,6 @@ int ensure_events(dem_ctx* ctx, size_t n)
         ctx->events.push_back(e);
     }
     return DEM_OK;
-}
-
-template <int NS>
-void run_one_step(dem_ctx* ctx, int64_t s, int64_t nsteps)
-{
-    // the first half-step and drift use the forces stored by the previous
-    // force pass; later ones are fused into the force kernel
-    if (s == 0) launch_kick<NS>(ctx, 0, 1);
-    ctx->prm.erase = 1;
-    ctx->prm.nt = (uint32_t)ctx->nt;
-    ctx->prm.alive_min = ctx->alive_min;
-    launch_rebuild<NS>(ctx);
-    launch_force<NS>(ctx, 1, s + 1 < nsteps ? KICK_BOTH : KICK_AFTER);
 }
 
 inline void advance_clock(dem_ctx* ctx)
@@ -2918,6 +2975,15 @@ std::vector<unsigned char> graph_key(dem_ctx* ctx)
     return k;
 }
 
+bool graphs_on(dem_ctx* ctx)
+{
+    if (ctx->graphs_off < 0) {
+        const char* env = std::getenv("DEM_STEP_GRAPH");
+        ctx->graphs_off = !(env && std::strcmp(env, "1") == 0);
+    }
+    return !ctx->graphs_off;
+}
+
 // A graph of two steady steps (rebuild launches, force pass with the fused
 // integration, counter advance; twice, so that the double buffers return to
 // their state at the start), captured on first use.  nullptr if capture is
@@ -2925,11 +2991,7 @@ std::vector<unsigned char> graph_key(dem_ctx* ctx)
 template <int NS>
 hipGraphExec_t step_graph(dem_ctx* ctx)
 {
-    if (ctx->graphs_off < 0) {
-        const char* env = std::getenv("DEM_STEP_GRAPH");
-        ctx->graphs_off = !(env && std::strcmp(env, "1") == 0);
-    }
-    if (ctx->graphs_off) return nullptr;
+    if (!graphs_on(ctx)) return nullptr;
     std::vector<unsigned char> key = graph_key<NS>(ctx);
     for (auto& g : ctx->graphs)
         if (g.exec && g.key == key) return g.exec;
@@ -2950,7 +3012,7 @@ hipGraphExec_t step_graph(dem_ctx* ctx)
     for (int k = 0; k < 2; ++k) {
         ctx->prm.erase = 1;
         launch_rebuild<NS>(ctx);
-        launch_force<NS>(ctx, 1, KICK_BOTH);
+        launch_force<NS>(ctx, 1, KICK_BOTH, (uint32_t)ctx->nt);
         hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(1), 0, ctx->stream, ctx->d_flags);
     }
     ctx->prm.step_dev = nullptr;
@@ -2969,14 +3031,126 @@ hipGraphExec_t step_graph(dem_ctx* ctx)
     return exec;
 }
 
+// The rebuild before the next force pass, if one is known to be needed.
+template <int NS>
+void rebuild_now(dem_ctx* ctx, int erase)
+{
+    ctx->prm.erase = erase;
+    ctx->prm.nt = (uint32_t)ctx->nt;
+    ctx->prm.alive_min = ctx->alive_min;
+    launch_rebuild<NS>(ctx);
+    ctx->since_rebuild = 0;
+}
+
+// n force passes, each fused with the integration that follows it (KICK_BOTH,
+// the last one `last_kick`); each advances the clock if they are steps.
+//
+// The rebuild kernels are launched only when a rebuild is due.  The device
+// decides that; a pass that finds its lists outdated does nothing, and neither
+// does any after it.  So the host launches passes ahead in batches, two of
+// them in flight, and looks at the word that the asking pass left in its
+// memory when a batch is over.  If one asked, it waits for what is in flight,
+// takes back the passes that did nothing, rebuilds and goes on.  (Nine rebuild
+// kernels per step that return at once cost 17 to 25 us per step: more than
+// the force pass of a few thousand spheres.)  Batches are an eighth of the
+// passes between rebuilds, 4 to 16: a rebuild then wastes about one and a half
+// batches of passes that return at once (2 to 3 us each) and one wait.
+template <int NS>
+int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
+{
+    const bool prof = ctx->profiling;
+    constexpr int kMaxBatch = 16;
+    // profiling: two events per pass in flight, two for the rebuild
+    if (prof) {
+        const int r = ensure_events(ctx, 4 * kMaxBatch + 2);
+        if (r) return r;
+    }
+    auto rebuild = [&]() -> int {
+        hipEvent_t* e = prof ? ctx->events.data() + 4 * kMaxBatch : nullptr;
+        if (prof) HIPCHK(hipEventRecord(e[0], ctx->stream));
+        rebuild_now<NS>(ctx, erase);
+        if (prof) {
+            HIPCHK(hipEventRecord(e[1], ctx->stream));
+            HIPCHK(hipEventSynchronize(e[1]));
+            float ms = 0;
+            HIPCHK(hipEventElapsedTime(&ms, e[0], e[1]));
+            ctx->t_rebuild += ms;
+        }
+        return DEM_OK;
+    };
+    int r;
+    if (ctx->lists_stale && (r = rebuild()) != 0) return r;
+    int64_t done = 0, sent = 0;  // passes known to have run, passes launched
+    int64_t end[2];              // the passes launched when a batch in flight ends
+    int oldest = 0, flying = 0;
+    auto finish = [&](int64_t upto) -> int {
+        if (prof)
+            for (int64_t s = done; s < upto; ++s) {
+                hipEvent_t* e = ctx->events.data() + 2 * (s % (2 * kMaxBatch));
+                float ms = 0;
+                HIPCHK(hipEventElapsedTime(&ms, e[0], e[1]));
+                ctx->t_force += ms;
+                if (steps) ++ctx->timed_steps;
+            }
+        for (int64_t s = done; s < upto && steps; ++s) advance_clock(ctx);
+        ctx->since_rebuild += upto - done;
+        done = upto;
+        return DEM_OK;
+    };
+    while (done < n) {
+        while (flying < 2 && sent < n) {
+            const int64_t to = std::min(n, sent + ctx->batch);
+            for (; sent < to; ++sent) {
+                hipEvent_t* e = prof ? ctx->events.data() + 2 * (sent % (2 * kMaxBatch)) : nullptr;
+                if (prof) HIPCHK(hipEventRecord(e[0], ctx->stream));
+                launch_force<NS>(ctx, erase, sent + 1 < n ? KICK_BOTH : last_kick,
+                                 (uint32_t)(ctx->nt + (steps ? sent - done : 0)));
+                if (prof) HIPCHK(hipEventRecord(e[1], ctx->stream));
+            }
+            const int b = (oldest + flying) & 1;
+            end[b] = to;
+            HIPCHK(hipEventRecord(ctx->batch_done[b], ctx->stream));
+            ++flying;
+        }
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipEventSynchronize(ctx->batch_done[oldest]));
+        if (__atomic_load_n(ctx->rebuild_word, __ATOMIC_ACQUIRE) == 0) {
+            if ((r = finish(end[oldest])) != 0) return r;
+            oldest ^= 1;
+            --flying;
+            continue;
+        }
+        // some pass asked for a rebuild: let the rest run out
+        if ((r = read_flags(ctx)) != 0) return r;
+        const uint32_t flag = (uint32_t)ctx->h_flags[F_REBUILD];
+        int64_t idle = 0;  // launched passes that did nothing
+        if (flag) idle = std::max<int64_t>(0, (int32_t)(rebuild_at(ctx->passes) - flag) / 2 + 1);
+        idle = std::min(idle, sent - done);
+        for (int64_t k = 0; k < idle; ++k, --sent) unlaunch_force<NS>(ctx, sent < n ? KICK_BOTH : last_kick);
+        if ((r = finish(sent)) != 0) return r;
+        flying = 0;
+        if (flag) {
+            ctx->batch = (int)std::min<int64_t>(kMaxBatch, std::max<int64_t>(4, ctx->since_rebuild / 8));
+            *ctx->rebuild_word = 0;
+            if ((r = rebuild()) != 0) return r;
+        }
+    }
+    return check_flags(ctx);
+}
+
 template <int NS>
 int run_steps(dem_ctx* ctx, int64_t nsteps)
 {
-    // profiling: events e[4s..4s+3] bracket kick | rebuild | force of step s
-    const bool prof = ctx->profiling;
-    if (!prof && nsteps >= 4) {
-        // the first step, pairs of steady steps from the graph, the rest
-        run_one_step<NS>(ctx, 0, nsteps);
+    if (nsteps == 0) return check_flags(ctx);
+    // the first half-step and drift use the forces stored by the previous
+    // force pass; later ones are fused into the force kernel
+    if (!ctx->profiling && nsteps >= 4 && graphs_on(ctx)) {
+        // the first step, pairs of steady steps from the graph, the rest;
+        // every step launches the rebuild kernels, which return at once when
+        // none is due
+        launch_kick<NS>(ctx, 0, 1);
+        rebuild_now<NS>(ctx, 1);
+        launch_force<NS>(ctx, 1, KICK_BOTH, (uint32_t)ctx->nt);
         advance_clock(ctx);
         int64_t s = 1;
         hipGraphExec_t g = step_graph<NS>(ctx);
@@ -2990,79 +3164,41 @@ int run_steps(dem_ctx* ctx, int64_t nsteps)
             }
         }
         for (; s < nsteps; ++s) {
-            run_one_step<NS>(ctx, s, nsteps);
+            rebuild_now<NS>(ctx, 1);
+            launch_force<NS>(ctx, 1, s + 1 < nsteps ? KICK_BOTH : KICK_AFTER, (uint32_t)ctx->nt);
             advance_clock(ctx);
         }
         HIPCHK(hipGetLastError());
         return check_flags(ctx);
     }
-    constexpr int64_t kChunk = 256;
-    for (int64_t s0 = 0; s0 < nsteps; s0 += kChunk) {
-        const int64_t n = std::min(kChunk, nsteps - s0);
-        if (prof) {
-            int r = ensure_events(ctx, (size_t)(4 * n + 2));
-            if (r) return r;
-        }
-        for (int64_t k = 0; k < n; ++k) {
-            const int64_t s = s0 + k;
-            if (prof) HIPCHK(hipEventRecord(ctx->events[4 * k], ctx->stream));
-            if (s == 0) launch_kick<NS>(ctx, 0, 1);
-            if (prof) HIPCHK(hipEventRecord(ctx->events[4 * k + 1], ctx->stream));
-            ctx->prm.erase = 1;
-            ctx->prm.nt = (uint32_t)ctx->nt;
-            ctx->prm.alive_min = ctx->alive_min;
-            launch_rebuild<NS>(ctx);
-            if (prof) HIPCHK(hipEventRecord(ctx->events[4 * k + 2], ctx->stream));
-            launch_force<NS>(ctx, 1, s + 1 < nsteps ? KICK_BOTH : KICK_AFTER);
-            if (prof) HIPCHK(hipEventRecord(ctx->events[4 * k + 3], ctx->stream));
-            advance_clock(ctx);
-        }
-        if (prof) {
-            HIPCHK(hipStreamSynchronize(ctx->stream));
-            for (int64_t k = 0; k < n; ++k) {
-                float a = 0, b = 0, c = 0;
-                HIPCHK(hipEventElapsedTime(&a, ctx->events[4 * k], ctx->events[4 * k + 1]));
-                HIPCHK(hipEventElapsedTime(&b, ctx->events[4 * k + 1], ctx->events[4 * k + 2]));
-                HIPCHK(hipEventElapsedTime(&c, ctx->events[4 * k + 2], ctx->events[4 * k + 3]));
-                ctx->t_kick += a;
-                ctx->t_rebuild += b;
-                ctx->t_force += c;
-            }
-            ctx->timed_steps += n;
-        }
+    if (ctx->profiling) {
+        int r = ensure_events(ctx, 2);
+        if (r) return r;
+        HIPCHK(hipEventRecord(ctx->events[0], ctx->stream));
+        launch_kick<NS>(ctx, 0, 1);
+        HIPCHK(hipEventRecord(ctx->events[1], ctx->stream));
+        HIPCHK(hipEventSynchronize(ctx->events[1]));
+        float ms = 0;
+        HIPCHK(hipEventElapsedTime(&ms, ctx->events[0], ctx->events[1]));
+        ctx->t_kick += ms;
+    } else {
+        launch_kick<NS>(ctx, 0, 1);
     }
-    HIPCHK(hipGetLastError());
-    return check_flags(ctx);
+    return run_passes<NS>(ctx, nsteps, 1, KICK_AFTER, true);
 }
 
 template <int NS>
 int run_forces(dem_ctx* ctx)
 {
-    ctx->prm.erase = 0;
-    ctx->prm.nt = (uint32_t)ctx->nt;
-    ctx->prm.alive_min = ctx->alive_min;
-    launch_rebuild<NS>(ctx);
-    launch_force<NS>(ctx, 0, KICK_NONE);
-    HIPCHK(hipGetLastError());
-    return check_flags(ctx);
+    return run_passes<NS>(ctx, 1, 0, KICK_NONE, false);
 }
 
 // The second part of one computeOneTimeStep (after actionsBeforeTimeStep):
-// the same launches as a step of run_steps, closing with the half-kick only.
+// a step of run_steps, closing with the half-kick only.
 template <int NS>
 int run_step_end(dem_ctx* ctx)
 {
-    ctx->prm.erase = 1;
-    ctx->prm.nt = (uint32_t)ctx->nt;
-    ctx->prm.alive_min = ctx->alive_min;
-    launch_rebuild<NS>(ctx);
-    launch_force<NS>(ctx, 1, KICK_AFTER);
-    ctx->time += ctx->dt;
-    ctx->nt += 1;
-    ctx->alive_min = (uint32_t)ctx->nt;
-    ctx->prm.alive_min = ctx->alive_min;
-    HIPCHK(hipGetLastError());
-    return check_flags(ctx);
+    return run_passes<NS>(ctx, 1, 1, KICK_AFTER, true);
 }
 
 template <int NS>
@@ -3086,6 +3222,11 @@ int run_set_kinematics(dem_ctx* ctx, const double* x, const double* v, const dou
                        dst[1], dst[2], dst[3]);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    // (the drift of dem_step_begin may have asked too)
+    if (__atomic_load_n(ctx->rebuild_word, __ATOMIC_ACQUIRE)) {
+        *ctx->rebuild_word = 0;
+        ctx->lists_stale = true;
+    }
     return DEM_OK;
 }
 
@@ -3174,15 +3315,16 @@ int append_in_place(dem_ctx* ctx, int64_t k, const uint32_t* id, const int32_t* 
     for (int a = 0; a < 3; ++a)
         HIPCHK(hipMemcpyAsync(udst[a] + n0, u.data() + a * k, sizeof(uint32_t) * k, hipMemcpyHostToDevice, s));
     const uint32_t end = (uint32_t)m;
-    const int one = 1;
+    const uint32_t at = rebuild_at(ctx->passes + 1);
     HIPCHK(hipMemcpyAsync(d.start + ctx->nbuckets, &end, sizeof end, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(ctx->d_flags + F_REBUILD, &one, sizeof one, hipMemcpyHostToDevice, s));
+    HIPCHK(hipMemcpyAsync(ctx->d_flags + F_REBUILD, &at, sizeof at, hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_clear_appended<NS>, dim3(grid_for(k)), dim3(kBlock), 0, s, d, (int)n0, (int)k);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s));
     ctx->n = m;
     ctx->prm.n = (int)m;
     ctx->max_id = id[k - 1];
+    ctx->lists_stale = true;
     return DEM_OK;
 }
 
@@ -3264,9 +3406,9 @@ int remove_in_place(dem_ctx* ctx, int64_t k, const int64_t* index)
                            (const uint32_t*)movers, (int)hc[1]);
     HIPCHK(hipGetLastError());
     const uint32_t end = (uint32_t)n_new;
-    const int one = 1;
+    const uint32_t due = rebuild_at(ctx->passes + 1);
     HIPCHK(hipMemcpyAsync(d.start + ctx->nbuckets, &end, sizeof end, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(ctx->d_flags + F_REBUILD, &one, sizeof one, hipMemcpyHostToDevice, s));
+    HIPCHK(hipMemcpyAsync(ctx->d_flags + F_REBUILD, &due, sizeof due, hipMemcpyHostToDevice, s));
     ctx->n = n_new;
     p.n = (int)n_new;
     launch_rebuild<NS>(ctx);
@@ -3472,6 +3614,9 @@ int dem_destroy(dem_ctx* ctx)
     if (ctx->d_region) (void)hipFree(ctx->d_region);
     if (ctx->d_remove) (void)hipFree(ctx->d_remove);
     for (hipEvent_t e : ctx->events) (void)hipEventDestroy(e);
+    for (hipEvent_t e : ctx->batch_done)
+        if (e) (void)hipEventDestroy(e);
+    if (ctx->rebuild_word) (void)hipHostFree(ctx->rebuild_word);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return DEM_OK;
@@ -3665,6 +3810,7 @@ static int upload_particles(dem_ctx* ctx, int64_t n, int64_t cap, const uint32_t
         return set_err(ctx, DEM_ERR_ARG, "upload_particles: bad arguments");
     if (cap > (int64_t)0x7FFFFFFF) return set_err(ctx, DEM_ERR_ARG, "too many particles");
     HIPCHK(hipSetDevice(ctx->device));
+    if (const int e = ensure_host_words(ctx)) return e;
     // --- validate and derive the grid on the host
     double rmin = 1e300, rmax = 0.0;
     double xmin[3] = {1e300, 1e300, 1e300}, xmax[3] = {-1e300, -1e300, -1e300};
@@ -3721,6 +3867,7 @@ static int upload_particles(dem_ctx* ctx, int64_t n, int64_t cap, const uint32_t
     p.inner = kInnerSkin * skin;
     p.inner_thr2 = (0.5 * p.inner) * (0.5 * p.inner) * 0.999;
     p.ref_unit = skin / 524288.0;
+    p.rebuild_word = ctx->rebuild_word;
     for (int a = 0; a < 3; ++a) p.axis_pb[a] = -1;
     for (int b = 0; b < p.nper; ++b) {
         p.axis_pb[ctx->periodic[b].axis] = b;
@@ -3862,7 +4009,9 @@ static int upload_particles(dem_ctx* ctx, int64_t n, int64_t cap, const uint32_t
     HIPCHK(hipMemcpy(dorig, orig.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(dspc, spc.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
     int flags[F_NUM] = {0};
-    flags[F_REBUILD] = 1;
+    flags[F_REBUILD] = (int)rebuild_at(ctx->passes + 1);
+    ctx->lists_stale = true;
+    *ctx->rebuild_word = 0;
     ctx->diverged = false;
     HIPCHK(hipMemcpy(ctx->d_flags, flags, sizeof flags, hipMemcpyHostToDevice));
     if (ctx->ns_springs == 9) {
@@ -3916,8 +4065,9 @@ int dem_upload_contacts(dem_ctx* ctx, int64_t n, const uint32_t* p_id, const uin
     HIPCHK(hipMemcpy(di, i_id, sizeof(uint32_t) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(dt, ts, sizeof(uint32_t) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(ds, spring, sizeof(double) * 9 * n, hipMemcpyHostToDevice));
-    int one = 1;
-    HIPCHK(hipMemcpy(ctx->d_flags + F_REBUILD, &one, sizeof one, hipMemcpyHostToDevice));
+    const uint32_t at = rebuild_at(ctx->passes + 1);
+    HIPCHK(hipMemcpy(ctx->d_flags + F_REBUILD, &at, sizeof at, hipMemcpyHostToDevice));
+    ctx->lists_stale = true;
     // uploaded records replace the current history
     if (ctx->ns_springs == 9)
         hipLaunchKernelGGL(k_zero_masks<9>, dim3(grid_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->d9, ctx->prm);

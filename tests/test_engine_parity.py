@@ -1006,3 +1006,35 @@ def test_force_pass_where_the_wavefronts_particles_change(n):
     for e in (g, o):
         e.step(3)
     assert_contacts_close(g, o)
+
+
+@pytest.mark.parametrize("skin", [0.004, 0.03])
+def test_batches_of_steps_equal_single_steps(skin):
+    """dem_step(n) launches its force passes ahead in batches of up to 16 and
+    takes back those that found their lists outdated: every n around the
+    batch sizes gives what n calls of dem_step(1) give, bit for bit, with the
+    same number of rebuilds and clock, and profiled as well."""
+    sc = S.mixture(n=200, seed=93, lx=5.0, ly=5.0, lz=5.0, inflate=1.08, vmax=3.0, laws="hvm",
+                   periodic=(True, False), walls=("bottom", "top"))
+    engines = [dem.Engine(skin=skin) for _ in range(3)]
+    for e in engines:
+        S.apply(e, sc)
+        e.compute_forces()
+    batched, single, profiled = engines
+    profiled.set_profiling(True)
+    total = 0
+    for n in (1, 2, 3, 7, 8, 9, 16, 17, 33, 60):
+        batched.step(n)
+        profiled.step(n)
+        for _ in range(n):
+            single.step(1)
+        total += n
+        a, s = batched.download(), batched.stats()
+        for e in (single, profiled):
+            b, t = e.download(), e.stats()
+            for k in a:
+                np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+            assert (t.n_steps, t.time, t.n_rebuilds, t.n_contacts) == (s.n_steps, s.time, s.n_rebuilds, s.n_contacts)
+    assert s.n_rebuilds > 3
+    assert profiled.stats().n_timed_steps == total
+    assert_contacts_equal(batched, single)
