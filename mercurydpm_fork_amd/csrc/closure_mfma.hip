@@ -3,15 +3,17 @@
 // (GELU hidden layers, linear output) with BF16 weights and FP32
 // accumulation, trained by full-batch Adam on FP32 master weights.
 //
-// The two 128 x 128 layers are GEMMs over the samples and run on the matrix
-// cores: v_mfma_f32_16x16x16_bf16 tiles, one 16 x 16 output tile per
-// wavefront, for the forward pass (Z = H W^T), the data gradient
-// (dH = dZ W) and the weight gradient (dW = dZ^T H, summed over the samples
-// in fixed chunks, then over the chunks in order, so the gradient is
-// deterministic).  The 4-wide input layer and the 2-wide output layer are too
-// narrow for a tile and run on the vector units with the same BF16 weights.
-// Activations fed to a matrix instruction are rounded to BF16 (round to
-// nearest even); pre-activations, GELU and every sum stay FP32.
+// The two 128 x 128 layers run on the matrix cores (v_mfma_f32_16x16x32_bf16)
+// in the forward pass (Z = H W^T), the data gradient (dH = dZ W) and the weight
+// gradient (dW = dZ^T H).  One kernel takes a tile of samples through the whole
+// network: inference keeps everything between the input and the output in
+// registers and LDS, training also goes back through the network and adds the
+// tile's gradient, and a second kernel sums the blocks' gradients in block
+// order (so they are the same bits on every run) and applies Adam.  The 4-wide
+// input layer and the 2-wide output layer are too narrow for a tile and run on
+// the vector units with the same BF16 weights.  Activations fed to a matrix
+// instruction are rounded to BF16 (round to nearest even); pre-activations,
+// GELU and every sum stay FP32.
 //
 // Parameter layout (FP32, one flat array): W1[128][4], b1[128],
 // W2[128][128], b2[128], W3[128][128], b3[128], W4[2][128], b4[2].
@@ -32,10 +34,10 @@ constexpr int oW1 = 0, oB1 = oW1 + kH * kIn, oW2 = oB1 + kH, oB2 = oW2 + kH * kH
               oB3 = oW3 + kH * kH, oW4 = oB3 + kH, oB4 = oW4 + kOut * kH, kP = oB4 + kOut;
 static_assert(kP == DEM_CLOSURE_PARAMS, "parameter count");
 constexpr int kBlock = 256;
-constexpr int kChunks = 16;  // sample chunks of the weight-gradient sums
 
-typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef uint16_t ushort4_t __attribute__((ext_vector_type(4)));
 
 // FP32 -> BF16, round to nearest even (finite values)
 __host__ __device__ inline uint16_t to_bf16(float f)
@@ -60,225 +62,471 @@ __device__ inline float gelu_grad(float z)
     return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-__global__ void k_cast_bf16(const float* __restrict__ p, uint16_t* __restrict__ q, int n)
+// BF16 weights as the kernels read them: W1 and W4 row-major, then W2 and W3
+// twice in operand order, for the forward pass (kF2, kF3: W as the second
+// operand of H W^T) and for the data gradient (kT2, kT3: of dZ W).  In operand
+// order the 8 values of lane l for tile t (16 columns of the product) and step
+// k (32 deep) lie at ((t * 4 + k) * 64 + l) * 8: a wavefront loads an operand
+// as one 1 KB run.
+constexpr int kTile = kH * kH;
+constexpr int kF2 = 1024, kF3 = kF2 + kTile, kT2 = kF3 + kTile, kT3 = kT2 + kTile, kPacked = kT3 + kTile;
+constexpr int kPackW1 = 0, kPackW4 = 512;
+static_assert(kH * kIn == 512 && kOut * kH == 256 && kH == 128, "packed layout");
+
+// where weight (row, column of the product) = (col, depth) lies in operand order
+__host__ __device__ inline int operand_at(int col, int depth)
+{
+    return (((col >> 4) * 4 + (depth >> 5)) * 64 + ((depth >> 3) & 3) * 16 + (col & 15)) * 8 + (depth & 7);
+}
+
+// parameter i, rounded, into the packed weights (biases are read as FP32)
+__device__ inline void pack_param(uint16_t* __restrict__ wb, int i, float v)
+{
+    const uint16_t h = to_bf16(v);
+    if (i < oB1) {
+        wb[kPackW1 + i] = h;
+    } else if (i >= oW2 && i < oB2) {
+        const int o = (i - oW2) / kH, k = (i - oW2) % kH;
+        wb[kF2 + operand_at(o, k)] = h;
+        wb[kT2 + operand_at(k, o)] = h;
+    } else if (i >= oW3 && i < oB3) {
+        const int o = (i - oW3) / kH, k = (i - oW3) % kH;
+        wb[kF3 + operand_at(o, k)] = h;
+        wb[kT3 + operand_at(k, o)] = h;
+    } else if (i >= oW4 && i < oB4) {
+        wb[kPackW4 + i - oW4] = h;
+    }
+}
+
+__global__ void k_pack(const float* __restrict__ p, uint16_t* __restrict__ wb)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) q[i] = to_bf16(p[i]);
+    if (i < kP) pack_param(wb, i, p[i]);
 }
 
-// input layer: Z1 = x W1^T + b1, H1 = bf16(gelu(Z1)); rows >= n are zero
-__global__ void k_layer_in(const float* __restrict__ x, const uint16_t* __restrict__ wb, const float* __restrict__ p,
-                           int n, int npad, float* __restrict__ z, uint16_t* __restrict__ h)
+// orders the LDS accesses of a wavefront's lanes
+__device__ inline void wave_sync()
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= npad * kH) return;
-    const int s = t / kH, o = t % kH;
-    float v = 0.0f;
-    if (s < n) {
-        v = p[oB1 + o];
-        for (int k = 0; k < kIn; ++k) v += x[kIn * s + k] * from_bf16(wb[oW1 + o * kIn + k]);
-    }
-    z[t] = v;
-    h[t] = s < n ? to_bf16(gelu(v)) : (uint16_t)0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// hidden layer on the matrix cores: Z = H_in W^T + b, H = bf16(gelu(Z)).
-// One wavefront per 16 x 16 tile (16 samples x 16 outputs), K = 128 in eight
-// 16-deep steps.  Operand layout of v_mfma_f32_16x16x16_bf16: lane l holds
-// A[l % 16][4 (l / 16) + j] and B[4 (l / 16) + j][l % 16] (j = 0..3) and
-// receives D[4 (l / 16) + i][l % 16] (i = 0..3).
-__global__ void __launch_bounds__(kBlock) k_layer_mfma(const uint16_t* __restrict__ hin,
-                                                       const uint16_t* __restrict__ w, const float* __restrict__ b,
-                                                       int n, int ntiles, float* __restrict__ z,
-                                                       uint16_t* __restrict__ h)
+// A wavefront holds 16 samples: lane l = 16 q + r has, of an activation, the
+// values of samples 4 q + i (i = 0..3) and columns 16 t + r (t = 0..7), which
+// is how a matrix instruction leaves its result.  As the next first operand
+// they go through LDS, 16 rows of kRow values (8 more than a row has, so that
+// the 16 rows of a load start in different banks).
+constexpr int kRow = kH + 8;
+constexpr int kCols = kH / 16, kDeep = kH / 32;
+typedef float Acts[kCols][4];
+
+__device__ inline void load_operand(const uint16_t* rows, int r, int q, bf16x8 a[kDeep])
 {
-    const int tile = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    if (tile >= ntiles) return;
-    const int lane = threadIdx.x & 63;
-    const int st = tile / (kH / 16), ot = tile % (kH / 16);
-    const int r = lane & 15, q = lane >> 4;
-    const short4_t* arow = (const short4_t*)(hin + (size_t)(st * 16 + r) * kH + 4 * q);
-    const short4_t* brow = (const short4_t*)(w + (size_t)(ot * 16 + r) * kH + 4 * q);
+#pragma unroll
+    for (int k = 0; k < kDeep; ++k) a[k] = *(const bf16x8*)(rows + r * kRow + 32 * k + 8 * q);
+}
+
+// columns 16 t .. 16 t + 15 of A times the packed second operand
+__device__ inline float4_t tile_product(const bf16x8 a[kDeep], const uint16_t* __restrict__ w, int t, int lane)
+{
     float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int kk = 0; kk < kH / 16; ++kk) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(arow[4 * kk], brow[4 * kk], acc, 0, 0, 0);
-    const int col = ot * 16 + r;
-    const float bias = b[col];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int s = st * 16 + 4 * q + i;
-        const float v = s < n ? acc[i] + bias : 0.0f;
-        z[(size_t)s * kH + col] = v;
-        h[(size_t)s * kH + col] = s < n ? to_bf16(gelu(v)) : (uint16_t)0;
-    }
+    for (int k = 0; k < kDeep; ++k)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k], *(const bf16x8*)(w + ((t * kDeep + k) * 64 + lane) * 8), acc,
+                                                      0, 0, 0);
+    return acc;
 }
 
-// output layer: y = H3 W4^T + b4
-__global__ void k_layer_out(const uint16_t* __restrict__ h, const uint16_t* __restrict__ wb,
-                            const float* __restrict__ p, int n, float* __restrict__ y)
+// input layer: z = x W1^T + b1 for the lane's samples (zero past the last)
+__device__ inline void layer_in(const float x[4][kIn], const bool live[4], const uint16_t* __restrict__ wb,
+                                const float* __restrict__ p, int r, Acts z)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * kOut) return;
-    const int s = t / kOut, o = t % kOut;
-    float v = p[oB4 + o];
-    for (int k = 0; k < kH; ++k) v += from_bf16(h[(size_t)s * kH + k]) * from_bf16(wb[oW4 + o * kH + k]);
-    y[t] = v;
-}
-
-// dY = 2 (y - t) / n (zero on padded rows) and the per-sample squared error
-__global__ void k_loss(const float* __restrict__ y, const float* __restrict__ tgt, int n, int npad,
-                       float* __restrict__ dy, float* __restrict__ se)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= npad) return;
-    float e2 = 0.0f;
-    for (int o = 0; o < kOut; ++o) {
-        const float e = s < n ? y[kOut * s + o] - tgt[kOut * s + o] : 0.0f;
-        dy[kOut * s + o] = 2.0f * e / (float)n;
-        e2 += e * e;
-    }
-    se[s] = e2;
-}
-
-// back through the output layer: dZ3 = (dY W4) * gelu'(Z3), FP32 and BF16
-__global__ void k_back_out(const float* __restrict__ dy, const uint16_t* __restrict__ wb,
-                           const float* __restrict__ z3, int npad, float* __restrict__ dz, uint16_t* __restrict__ dzb)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= npad * kH) return;
-    const int s = t / kH, k = t % kH;
-    float g = 0.0f;
-    for (int o = 0; o < kOut; ++o) g += dy[kOut * s + o] * from_bf16(wb[oW4 + o * kH + k]);
-    g *= gelu_grad(z3[t]);
-    dz[t] = g;
-    dzb[t] = to_bf16(g);
-}
-
-// data gradient on the matrix cores: dH = dZ W, then dZ_prev = dH *
-// gelu'(Z_prev) (FP32 and BF16).  A = dZ (samples x outputs), B = W
-// (outputs x inputs).
-__global__ void __launch_bounds__(kBlock) k_back_data_mfma(const uint16_t* __restrict__ dzb,
-                                                           const uint16_t* __restrict__ w,
-                                                           const float* __restrict__ zprev, int ntiles,
-                                                           float* __restrict__ dzp, uint16_t* __restrict__ dzpb)
-{
-    const int tile = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    if (tile >= ntiles) return;
-    const int lane = threadIdx.x & 63;
-    const int st = tile / (kH / 16), kt = tile % (kH / 16);
-    const int r = lane & 15, q = lane >> 4;
-    const short4_t* arow = (const short4_t*)(dzb + (size_t)(st * 16 + r) * kH + 4 * q);
-    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int oo = 0; oo < kH / 16; ++oo) {
-        short4_t bv;
+    for (int t = 0; t < kCols; ++t) {
+        const int col = 16 * t + r;
+        const ushort4_t w = *(const ushort4_t*)(wb + kPackW1 + col * kIn);
+        const float bias = p[oB1 + col];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bv[j] = (short)w[(size_t)(oo * 16 + 4 * q + j) * kH + kt * 16 + r];
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(arow[4 * oo], bv, acc, 0, 0, 0);
-    }
-    const int col = kt * 16 + r;
+        for (int i = 0; i < 4; ++i) {
+            float v = bias;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const size_t at = (size_t)(st * 16 + 4 * q + i) * kH + col;
-        const float g = acc[i] * gelu_grad(zprev[at]);
-        dzp[at] = g;
-        dzpb[at] = to_bf16(g);
-    }
-}
-
-// weight gradient on the matrix cores, per sample chunk: dW_c = dZ^T H over
-// the chunk's samples.  A[o][s] = dZ[s][o], B[s][k] = H[s][k]; one
-// wavefront per (16 x 16 tile of dW, chunk).
-__global__ void __launch_bounds__(kBlock) k_back_weight_mfma(const uint16_t* __restrict__ dzb,
-                                                             const uint16_t* __restrict__ h, int nst,
-                                                             float* __restrict__ part)
-{
-    const int item = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    constexpr int tiles = (kH / 16) * (kH / 16);
-    if (item >= tiles * kChunks) return;
-    const int c = item / tiles, tile = item % tiles;
-    const int ot = tile / (kH / 16), kt = tile % (kH / 16);
-    const int lane = threadIdx.x & 63;
-    const int r = lane & 15, q = lane >> 4;
-    const int per = (nst + kChunks - 1) / kChunks;
-    const int s0 = c * per, s1 = min(nst, s0 + per);
-    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int st = s0; st < s1; ++st) {
-        short4_t av, bv;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t row = (size_t)(st * 16 + 4 * q + j) * kH;
-            av[j] = (short)dzb[row + ot * 16 + r];
-            bv[j] = (short)h[row + kt * 16 + r];
+            for (int k = 0; k < kIn; ++k) v += x[i][k] * from_bf16(w[k]);
+            z[t][i] = live[i] ? v : 0.0f;
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
     }
-    float* out = part + (size_t)c * kH * kH;
+}
+
+// Inference: 16 samples per wavefront and turn, the 128 x 128 weights of both
+// layers in LDS (64 KB in operand order), nothing between x and y in memory.
+// Bound by the GELUs (384 erf per sample; the matrix products take an eighth of
+// the time).  1,000,003 samples: 0.31 ms; with a kernel per layer and the
+// activations through memory 2.26 ms.  Non-finite inputs are reported in *bad.
+constexpr int kInferWaves = 8;
+__global__ void __launch_bounds__(64 * kInferWaves) k_infer(const float* __restrict__ x, int n,
+                                                            const float* __restrict__ p,
+                                                            const uint16_t* __restrict__ wb, float* __restrict__ y,
+                                                            int* bad)
+{
+    __shared__ __align__(16) uint16_t w[2 * kTile];
+    __shared__ __align__(16) uint16_t act[kInferWaves][16 * kRow];
+    for (int i = threadIdx.x; i < 2 * kTile / 8; i += 64 * kInferWaves)
+        ((uint4*)w)[i] = ((const uint4*)(wb + kF2))[i];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    uint16_t* rows = act[wave];
+    const int tiles = (n + 15) / 16;
+    for (int tile = blockIdx.x * kInferWaves + wave; tile < tiles; tile += gridDim.x * kInferWaves) {
+        const int s0 = tile * 16;
+        float xs[4][kIn];
+        bool live[4];
+        bool finite = true;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[(size_t)(ot * 16 + 4 * q + i) * kH + kt * 16 + r] = acc[i];
-}
-
-// the chunk partials of a weight gradient summed in chunk order
-__global__ void k_sum_chunks(const float* __restrict__ part, int len, float* __restrict__ out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= len) return;
-    float s = 0.0f;
-    for (int c = 0; c < kChunks; ++c) s += part[(size_t)c * len + i];
-    out[i] = s;
-}
-
-// column sums over the samples (bias gradients) and the small weight
-// gradients of the input and output layers, one thread per entry, samples
-// in order: out[o] = sum_s a[s][o] (bias, kind 0); dW1[o][k] = sum_s dZ1[s][o]
-// x[s][k] (kind 1); dW4[o][k] = sum_s dY[s][o] H3[s][k] (kind 2)
-__global__ void k_small_grads(const float* __restrict__ dz1, const float* __restrict__ dz2,
-                              const float* __restrict__ dz3, const float* __restrict__ dy,
-                              const float* __restrict__ x, const uint16_t* __restrict__ h3, int n,
-                              float* __restrict__ g)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < kH * kIn) {  // dW1
-        const int o = t / kIn, k = t % kIn;
-        float s = 0.0f;
-        for (int i = 0; i < n; ++i) s += dz1[(size_t)i * kH + o] * x[kIn * i + k];
-        g[oW1 + t] = s;
-    } else if (t < kH * kIn + 3 * kH) {  // b1, b2, b3
-        const int u = t - kH * kIn, l = u / kH, o = u % kH;
-        const float* a = l == 0 ? dz1 : (l == 1 ? dz2 : dz3);
-        float s = 0.0f;
-        for (int i = 0; i < n; ++i) s += a[(size_t)i * kH + o];
-        g[(l == 0 ? oB1 : (l == 1 ? oB2 : oB3)) + o] = s;
-    } else if (t < kH * kIn + 3 * kH + kOut * kH) {  // dW4
-        const int u = t - kH * kIn - 3 * kH, o = u / kH, k = u % kH;
-        float s = 0.0f;
-        for (int i = 0; i < n; ++i) s += dy[kOut * i + o] * from_bf16(h3[(size_t)i * kH + k]);
-        g[oW4 + u] = s;
-    } else if (t < kH * kIn + 3 * kH + kOut * kH + kOut) {  // b4
-        const int o = t - kH * kIn - 3 * kH - kOut * kH;
-        float s = 0.0f;
-        for (int i = 0; i < n; ++i) s += dy[kOut * i + o];
-        g[oB4 + o] = s;
+        for (int i = 0; i < 4; ++i) {
+            const int s = s0 + 4 * q + i;
+            live[i] = s < n;
+            const float4 v = live[i] ? ((const float4*)x)[s] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            xs[i][0] = v.x;
+            xs[i][1] = v.y;
+            xs[i][2] = v.z;
+            xs[i][3] = v.w;
+            finite = finite && isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w);
+        }
+        if (!finite) *bad = 1;
+        Acts z;
+        layer_in(xs, live, wb, p, r, z);
+#pragma unroll
+        for (int layer = 0; layer < 2; ++layer) {
+            wave_sync();
+#pragma unroll
+            for (int t = 0; t < kCols; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) rows[(4 * q + i) * kRow + 16 * t + r] = to_bf16(gelu(z[t][i]));
+            wave_sync();
+            bf16x8 a[kDeep];
+            load_operand(rows, r, q, a);
+#pragma unroll
+            for (int t = 0; t < kCols; ++t) {
+                const float bias = p[(layer ? oB3 : oB2) + 16 * t + r];
+                const float4_t acc = tile_product(a, w + layer * kTile, t, lane);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) z[t][i] = acc[i] + bias;
+            }
+        }
+        float out[4][kOut] = {};
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+            const float w0 = from_bf16(wb[kPackW4 + 16 * t + r]), w1 = from_bf16(wb[kPackW4 + kH + 16 * t + r]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float h = from_bf16(to_bf16(gelu(z[t][i])));
+                out[i][0] += h * w0;
+                out[i][1] += h * w1;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int o = 0; o < kOut; ++o) {
+                float v = out[i][o];
+                for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m, 64);
+                out[i][o] = v + p[oB4 + o];
+            }
+        if (r == 0)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (live[i]) ((float2*)y)[s0 + 4 * q + i] = make_float2(out[i][0], out[i][1]);
     }
 }
 
-__global__ void k_sum_loss(const float* __restrict__ se, int n, float* __restrict__ loss)
+// Forward and backward through the network for tiles of 64 samples, 16 per
+// wavefront, and the block's share of the loss and of every gradient, written
+// to row blockIdx.x of part (kP gradients, then the sum of squared errors).
+//
+// What crosses samples, the weight gradients dZ^T H, needs its operands sample
+// by sample: activations and their gradients are therefore also kept in LDS
+// column by column (kCol samples a column), where the four values that a lane
+// holds of one column are neighbours.  After a tile the four wavefronts share
+// the 64 tiles of each weight gradient, 16 apiece, which stay in registers over
+// the block's tiles (one block per CU: 512 registers a lane).  The pre-
+// activations stay in registers from the forward to the backward pass.
+//
+// Bound by the chain of GELUs and their derivatives that a wavefront evaluates
+// (768 erf per sample), one wavefront per SIMD.  14,188 samples: 77 us, and 9 us
+// for the sums and the Adam step; an epoch of the sixteen kernels this replaces
+// took 4.6 ms, of which 3.9 ms were the sums over the samples by one thread per
+// entry and 0.65 ms the loss by one thread.
+constexpr int kTrainWaves = 4, kTrainTile = 16 * kTrainWaves;
+constexpr int kCol = kTrainTile + 8;
+constexpr int kPart = kP + 1;
+
+// the lane's values of an activation, rounded, into rows and columns
+__device__ inline void put_rows(uint16_t* rows, int r, int q, int t, const uint16_t h[4])
 {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    float s = 0.0f;
-    for (int i = 0; i < n; ++i) s += se[i];
-    loss[0] = s / (float)n;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rows[(4 * q + i) * kRow + 16 * t + r] = h[i];
+}
+__device__ inline void put_column(uint16_t* cols, int wave, int r, int q, int t, const uint16_t h[4])
+{
+    *(ushort4_t*)(cols + (16 * t + r) * kCol + 16 * wave + 4 * q) = ushort4_t{h[0], h[1], h[2], h[3]};
 }
 
-__global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                       const float* __restrict__ g, int n, float lr, float c1, float c2)
+// += the weight gradient dZ^T H of a block's tile, rows 32 wave .. 32 wave + 31
+__device__ inline void add_weight_grad(const uint16_t* dz, const uint16_t* h, int wave, int r, int q,
+                                       float4_t acc[2][kCols])
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    m[i] = 0.9f * m[i] + 0.1f * gi;
-    v[i] = 0.999f * v[i] + 0.001f * gi * gi;
-    p[i] -= lr * (m[i] / c1) / (sqrtf(v[i] / c2) + 1e-8f);
+#pragma unroll
+    for (int k = 0; k < kTrainTile / 32; ++k) {
+        bf16x8 a[2];
+#pragma unroll
+        for (int o = 0; o < 2; ++o) a[o] = *(const bf16x8*)(dz + (32 * wave + 16 * o + r) * kCol + 32 * k + 8 * q);
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+            const bf16x8 b = *(const bf16x8*)(h + (16 * t + r) * kCol + 32 * k + 8 * q);
+#pragma unroll
+            for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[o], b, acc[o][t], 0, 0, 0);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(64 * kTrainWaves, 1) k_train_tile(const float* __restrict__ x,
+                                                                    const float* __restrict__ tgt, int n,
+                                                                    const float* __restrict__ p,
+                                                                    const uint16_t* __restrict__ packed,
+                                                                    float* __restrict__ part)
+{
+    __shared__ __align__(16) uint16_t act[kTrainWaves][16 * kRow];
+    __shared__ __align__(16) uint16_t h1[kH * kCol], h2[kH * kCol], e2[kH * kCol], e3[kH * kCol];
+    // gradients that a wavefront sums over its own samples: W1, b1, b2, b3, W4,
+    // b4, loss (a block's four rows of them are added in order at the end)
+    constexpr int sW1 = 0, sB1 = sW1 + kH * kIn, sB2 = sB1 + kH, sB3 = sB2 + kH, sW4 = sB3 + kH, sB4 = sW4 + kOut * kH,
+                  sLoss = sB4 + kOut, kSmall = sLoss + 1;
+    __shared__ float small[kTrainWaves][kSmall];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    uint16_t* rows = act[wave];
+    float4_t g2[2][kCols] = {}, g3[2][kCols] = {};
+    float* mine = small[wave];
+    for (int i = lane; i < kSmall; i += 64) mine[i] = 0.0f;
+    // the sum of v over the four sample groups q, added to a small gradient
+    auto add_small = [&](int at, float v) {
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        if (q == 0) mine[at] += v;
+    };
+    const float two_over_n = 2.0f / (float)n;
+    const int tiles = (n + kTrainTile - 1) / kTrainTile;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int s0 = tile * kTrainTile + 16 * wave;
+        // (hidden from the compiler, which would load all the weights once, before
+        // the loop, and spill them)
+        const uint16_t* wb = packed;
+        asm volatile("" : "+s"(wb));
+        float xs[4][kIn];
+        bool live[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int s = s0 + 4 * q + i;
+            live[i] = s < n;
+            const float4 v = live[i] ? ((const float4*)x)[s] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            xs[i][0] = v.x;
+            xs[i][1] = v.y;
+            xs[i][2] = v.z;
+            xs[i][3] = v.w;
+        }
+        // forward
+        Acts z1, z2, z3;
+        uint16_t h[4];
+        layer_in(xs, live, wb, p, r, z1);
+        wave_sync();
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h[i] = live[i] ? to_bf16(gelu(z1[t][i])) : (uint16_t)0;
+            put_rows(rows, r, q, t, h);
+            put_column(h1, wave, r, q, t, h);
+        }
+        wave_sync();
+        bf16x8 a[kDeep];
+        load_operand(rows, r, q, a);
+        wave_sync();
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+            const float bias = p[oB2 + 16 * t + r];
+            const float4_t acc = tile_product(a, wb + kF2, t, lane);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                z2[t][i] = live[i] ? acc[i] + bias : 0.0f;
+                h[i] = live[i] ? to_bf16(gelu(z2[t][i])) : (uint16_t)0;
+            }
+            put_rows(rows, r, q, t, h);
+            put_column(h2, wave, r, q, t, h);
+        }
+        wave_sync();
+        load_operand(rows, r, q, a);
+        wave_sync();
+        float out[4][kOut] = {};
+        uint16_t h3[kCols][4];
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+            const float bias = p[oB3 + 16 * t + r];
+            const float4_t acc = tile_product(a, wb + kF3, t, lane);
+            const float w0 = from_bf16(wb[kPackW4 + 16 * t + r]), w1 = from_bf16(wb[kPackW4 + kH + 16 * t + r]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                z3[t][i] = live[i] ? acc[i] + bias : 0.0f;
+                h3[t][i] = live[i] ? to_bf16(gelu(z3[t][i])) : (uint16_t)0;
+                out[i][0] += from_bf16(h3[t][i]) * w0;
+                out[i][1] += from_bf16(h3[t][i]) * w1;
+            }
+        }
+        // loss: dY = 2 (y - t) / n
+        float dy[4][kOut], loss = 0.0f, gb4[kOut] = {};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int o = 0; o < kOut; ++o) {
+                float v = out[i][o];
+                for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m, 64);
+                const float e = live[i] ? v + p[oB4 + o] - tgt[kOut * (s0 + 4 * q + i) + o] : 0.0f;
+                dy[i][o] = e * two_over_n;
+                gb4[o] += dy[i][o];
+                loss += e * e;
+            }
+        // (the same in the 16 lanes of a group: lane 0 adds them)
+        for (int m = 16; m < 64; m <<= 1) {
+            gb4[0] += __shfl_xor(gb4[0], m, 64);
+            gb4[1] += __shfl_xor(gb4[1], m, 64);
+            loss += __shfl_xor(loss, m, 64);
+        }
+        if (lane == 0) {
+            mine[sB4] += gb4[0];
+            mine[sB4 + 1] += gb4[1];
+            mine[sLoss] += loss;
+        }
+        // back through the output layer
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+            const float w0 = from_bf16(wb[kPackW4 + 16 * t + r]), w1 = from_bf16(wb[kPackW4 + kH + 16 * t + r]);
+            float gw0 = 0.0f, gw1 = 0.0f, gb = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float hv = from_bf16(h3[t][i]);
+                gw0 += dy[i][0] * hv;
+                gw1 += dy[i][1] * hv;
+                const float dz = (dy[i][0] * w0 + dy[i][1] * w1) * gelu_grad(z3[t][i]);
+                gb += dz;
+                h[i] = to_bf16(dz);
+            }
+            add_small(sW4 + 16 * t + r, gw0);
+            add_small(sW4 + kH + 16 * t + r, gw1);
+            add_small(sB3 + 16 * t + r, gb);
+            put_rows(rows, r, q, t, h);
+            put_column(e3, wave, r, q, t, h);
+        }
+        // dZ2 = (dZ3 W3) * gelu'(Z2), dZ1 = (dZ2 W2) * gelu'(Z1)
+        wave_sync();
+        load_operand(rows, r, q, a);
+        wave_sync();
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+            const float4_t acc = tile_product(a, wb + kT3, t, lane);
+            float gb = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float dz = acc[i] * gelu_grad(z2[t][i]);
+                gb += dz;
+                h[i] = to_bf16(dz);
+            }
+            add_small(sB2 + 16 * t + r, gb);
+            put_rows(rows, r, q, t, h);
+            put_column(e2, wave, r, q, t, h);
+        }
+        wave_sync();
+        load_operand(rows, r, q, a);
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) {
+            const float4_t acc = tile_product(a, wb + kT2, t, lane);
+            float gb = 0.0f, gw[kIn] = {};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float dz = acc[i] * gelu_grad(z1[t][i]);
+                gb += dz;
+#pragma unroll
+                for (int k = 0; k < kIn; ++k) gw[k] += dz * xs[i][k];
+            }
+            add_small(sB1 + 16 * t + r, gb);
+#pragma unroll
+            for (int k = 0; k < kIn; ++k) add_small(sW1 + (16 * t + r) * kIn + k, gw[k]);
+        }
+        __syncthreads();
+        add_weight_grad(e3, h2, wave, r, q, g3);
+        add_weight_grad(e2, h1, wave, r, q, g2);
+        __syncthreads();
+    }
+    float* row = part + (size_t)blockIdx.x * kPart;
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int t = 0; t < kCols; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int at = (32 * wave + 16 * o + 4 * q + i) * kH + 16 * t + r;
+                row[oW2 + at] = g2[o][t][i];
+                row[oW3 + at] = g3[o][t][i];
+            }
+    // the wavefronts' small gradients in order
+    __syncthreads();
+    for (int i = threadIdx.x; i < kSmall; i += 64 * kTrainWaves) {
+        float v = small[0][i];
+#pragma unroll
+        for (int w = 1; w < kTrainWaves; ++w) v += small[w][i];
+        const int at = i < sB1   ? oW1 + i - sW1
+                       : i < sB2 ? oB1 + i - sB1
+                       : i < sB3 ? oB2 + i - sB2
+                       : i < sW4 ? oB3 + i - sB3
+                       : i < sB4 ? oW4 + i - sW4
+                                 : oB4 + i - sB4;
+        row[at] = v;
+    }
+}
+
+// The blocks' gradients summed (four quarters of the rows, each in order, then
+// in order) into g and the mean squared error into loss; with lr > 0 the Adam
+// step and the packed weights of the next pass as well.
+constexpr int kSumWays = 4;
+__global__ void __launch_bounds__(kBlock) k_sum_and_step(const float* __restrict__ part, int rows, int n,
+                                                         float* __restrict__ g, float* __restrict__ loss,
+                                                         float* __restrict__ p, float* __restrict__ m,
+                                                         float* __restrict__ v, uint16_t* __restrict__ wb, float lr,
+                                                         float c1, float c2)
+{
+    __shared__ float red[kSumWays][kBlock / kSumWays];
+    const int way = threadIdx.x / (kBlock / kSumWays), at = threadIdx.x % (kBlock / kSumWays);
+    const int i = blockIdx.x * (kBlock / kSumWays) + at;
+    const int per = (rows + kSumWays - 1) / kSumWays;
+    const int r0 = way * per, r1 = min(rows, r0 + per);
+    float s = 0.0f;
+    if (i < kPart)
+#pragma unroll 8
+        for (int r = r0; r < r1; ++r) s += part[(size_t)r * kPart + i];
+    red[way][at] = s;
+    __syncthreads();
+    if (way != 0 || i >= kPart) return;
+#pragma unroll
+    for (int w = 1; w < kSumWays; ++w) s += red[w][at];
+    if (i == kP) {
+        loss[0] = s / (float)n;
+        return;
+    }
+    g[i] = s;
+    if (!(lr > 0.0f)) return;
+    m[i] = 0.9f * m[i] + 0.1f * s;
+    v[i] = 0.999f * v[i] + 0.001f * s * s;
+    const float q = p[i] - lr * (m[i] / c1) / (sqrtf(v[i] / c2) + 1e-8f);
+    p[i] = q;
+    pack_param(wb, i, q);
 }
 
 inline unsigned blocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -291,11 +539,16 @@ struct dem_closure {
     float *p = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;
     uint16_t* wb = nullptr;
     int64_t step = 0;
-    // per-sample buffers, grown on demand
+    // sample buffers, grown on demand
     int64_t cap = 0;
-    float *x = nullptr, *t = nullptr, *y = nullptr, *dy = nullptr, *se = nullptr, *loss = nullptr;
-    float *z1 = nullptr, *z2 = nullptr, *z3 = nullptr, *d1 = nullptr, *d2 = nullptr, *d3 = nullptr, *part = nullptr;
-    uint16_t *h1 = nullptr, *h2 = nullptr, *h3 = nullptr, *e1 = nullptr, *e2 = nullptr, *e3 = nullptr;
+    float *x = nullptr, *t = nullptr, *y = nullptr;
+    // the training blocks' gradients, and the loss
+    int64_t part_rows = 0;
+    float *part = nullptr, *loss = nullptr;
+    // pinned host memory that the kernels read and write directly: the inputs
+    // and outputs of a small forward call, and the non-finite flag
+    float *hx = nullptr, *hy = nullptr;
+    int* bad = nullptr;
 };
 
 namespace {
@@ -305,76 +558,73 @@ namespace {
         if ((expr) != hipSuccess) return DEM_ERR_DEVICE; \
     } while (0)
 
+// forward calls of up to this many samples go through pinned memory: two
+// copies of a few KB each cost more than the kernel
+constexpr int64_t kSmallCall = 2048;
+constexpr int kMaxTrainBlocks = 256;  // one per CU
+
 void free_samples(dem_closure* c)
 {
-    for (void* a : {(void*)c->x, (void*)c->t, (void*)c->y, (void*)c->dy, (void*)c->se, (void*)c->loss, (void*)c->z1,
-                    (void*)c->z2, (void*)c->z3, (void*)c->d1, (void*)c->d2, (void*)c->d3, (void*)c->part,
-                    (void*)c->h1, (void*)c->h2, (void*)c->h3, (void*)c->e1, (void*)c->e2, (void*)c->e3})
+    for (void* a : {(void*)c->x, (void*)c->t, (void*)c->y})
         if (a) (void)hipFree(a);
-    c->x = c->t = c->y = c->dy = c->se = c->loss = c->z1 = c->z2 = c->z3 = c->d1 = c->d2 = c->d3 = c->part = nullptr;
-    c->h1 = c->h2 = c->h3 = c->e1 = c->e2 = c->e3 = nullptr;
+    c->x = c->t = c->y = nullptr;
     c->cap = 0;
 }
 
 int ensure(dem_closure* c, int64_t n)
 {
-    const int64_t npad = (n + 15) / 16 * 16;
-    if (npad <= c->cap) return DEM_OK;
+    if (n <= c->cap) return DEM_OK;
     CCHK(hipStreamSynchronize(c->stream));
     free_samples(c);
-    const size_t a = (size_t)npad * kH;
-    CCHK(hipMalloc(&c->x, sizeof(float) * kIn * npad));
-    CCHK(hipMalloc(&c->t, sizeof(float) * kOut * npad));
-    CCHK(hipMalloc(&c->y, sizeof(float) * kOut * npad));
-    CCHK(hipMalloc(&c->dy, sizeof(float) * kOut * npad));
-    CCHK(hipMalloc(&c->se, sizeof(float) * npad));
-    CCHK(hipMalloc(&c->loss, sizeof(float)));
-    for (float** b : {&c->z1, &c->z2, &c->z3, &c->d1, &c->d2, &c->d3}) CCHK(hipMalloc(b, sizeof(float) * a));
-    for (uint16_t** b : {&c->h1, &c->h2, &c->h3, &c->e1, &c->e2, &c->e3}) CCHK(hipMalloc(b, sizeof(uint16_t) * a));
-    CCHK(hipMalloc(&c->part, sizeof(float) * kChunks * kH * kH));
-    c->cap = npad;
+    CCHK(hipMalloc(&c->x, sizeof(float) * kIn * n));
+    CCHK(hipMalloc(&c->t, sizeof(float) * kOut * n));
+    CCHK(hipMalloc(&c->y, sizeof(float) * kOut * n));
+    c->cap = n;
     return DEM_OK;
 }
 
-// the forward pass of the samples in c->x (n of them, npad rows)
-void forward(dem_closure* c, int n)
+int train_blocks(int64_t n)
 {
-    const int npad = (n + 15) / 16 * 16;
-    const int ntiles = (npad / 16) * (kH / 16);
-    hipLaunchKernelGGL(k_cast_bf16, dim3(blocks(kP)), dim3(kBlock), 0, c->stream, c->p, c->wb, kP);
-    hipLaunchKernelGGL(k_layer_in, dim3(blocks((int64_t)npad * kH)), dim3(kBlock), 0, c->stream, c->x, c->wb, c->p, n,
-                       npad, c->z1, c->h1);
-    hipLaunchKernelGGL(k_layer_mfma, dim3((ntiles + 3) / 4), dim3(kBlock), 0, c->stream, c->h1, c->wb + oW2,
-                       c->p + oB2, n, ntiles, c->z2, c->h2);
-    hipLaunchKernelGGL(k_layer_mfma, dim3((ntiles + 3) / 4), dim3(kBlock), 0, c->stream, c->h2, c->wb + oW3,
-                       c->p + oB3, n, ntiles, c->z3, c->h3);
-    hipLaunchKernelGGL(k_layer_out, dim3(blocks((int64_t)n * kOut)), dim3(kBlock), 0, c->stream, c->h3, c->wb, c->p,
-                       n, c->y);
+    const int64_t tiles = (n + kTrainTile - 1) / kTrainTile;
+    return (int)(tiles < kMaxTrainBlocks ? tiles : kMaxTrainBlocks);
 }
 
-// loss and gradient (into c->g) of the samples in c->x / c->t
-void backward(dem_closure* c, int n)
+int ensure_part(dem_closure* c, int64_t n)
 {
-    const int npad = (n + 15) / 16 * 16;
-    const int ntiles = (npad / 16) * (kH / 16);
-    const int nst = npad / 16;
-    hipLaunchKernelGGL(k_loss, dim3(blocks(npad)), dim3(kBlock), 0, c->stream, c->y, c->t, n, npad, c->dy, c->se);
-    hipLaunchKernelGGL(k_back_out, dim3(blocks((int64_t)npad * kH)), dim3(kBlock), 0, c->stream, c->dy, c->wb, c->z3,
-                       npad, c->d3, c->e3);
-    const unsigned wblocks = (unsigned)(((kH / 16) * (kH / 16) * kChunks + 3) / 4);
-    // layer 3: dW3 = dZ3^T H2, dZ2 = (dZ3 W3) * gelu'(Z2)
-    hipLaunchKernelGGL(k_back_weight_mfma, dim3(wblocks), dim3(kBlock), 0, c->stream, c->e3, c->h2, nst, c->part);
-    hipLaunchKernelGGL(k_sum_chunks, dim3(blocks(kH * kH)), dim3(kBlock), 0, c->stream, c->part, kH * kH, c->g + oW3);
-    hipLaunchKernelGGL(k_back_data_mfma, dim3((ntiles + 3) / 4), dim3(kBlock), 0, c->stream, c->e3, c->wb + oW3,
-                       c->z2, ntiles, c->d2, c->e2);
-    // layer 2: dW2 = dZ2^T H1, dZ1 = (dZ2 W2) * gelu'(Z1)
-    hipLaunchKernelGGL(k_back_weight_mfma, dim3(wblocks), dim3(kBlock), 0, c->stream, c->e2, c->h1, nst, c->part);
-    hipLaunchKernelGGL(k_sum_chunks, dim3(blocks(kH * kH)), dim3(kBlock), 0, c->stream, c->part, kH * kH, c->g + oW2);
-    hipLaunchKernelGGL(k_back_data_mfma, dim3((ntiles + 3) / 4), dim3(kBlock), 0, c->stream, c->e2, c->wb + oW2,
-                       c->z1, ntiles, c->d1, c->e1);
-    hipLaunchKernelGGL(k_small_grads, dim3(blocks(kH * kIn + 3 * kH + kOut * kH + kOut)), dim3(kBlock), 0, c->stream,
-                       c->d1, c->d2, c->d3, c->dy, c->x, c->h3, n, c->g);
-    hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(1), 0, c->stream, c->se, n, c->loss);
+    const int64_t rows = train_blocks(n);
+    if (rows <= c->part_rows) return DEM_OK;
+    CCHK(hipStreamSynchronize(c->stream));
+    if (c->part) (void)hipFree(c->part);
+    c->part = nullptr;
+    c->part_rows = 0;
+    CCHK(hipMalloc(&c->part, sizeof(float) * kPart * rows));
+    c->part_rows = rows;
+    return DEM_OK;
+}
+
+// the packed weights follow the parameters: after set_params here, after an
+// Adam step in k_sum_and_step
+void pack(dem_closure* c)
+{
+    hipLaunchKernelGGL(k_pack, dim3(blocks(kP)), dim3(kBlock), 0, c->stream, c->p, c->wb);
+}
+
+void forward(dem_closure* c, int n, const float* x, float* y)
+{
+    const int tiles = (n + 16 * kInferWaves - 1) / (16 * kInferWaves);
+    hipLaunchKernelGGL(k_infer, dim3(tiles < 256 ? tiles : 256), dim3(64 * kInferWaves), 0, c->stream, x, n, c->p, c->wb,
+                       y, c->bad);
+}
+
+// loss and gradient (into c->g) of the samples in c->x / c->t; lr > 0: and the
+// Adam step
+void backward(dem_closure* c, int n, float lr, float c1, float c2)
+{
+    const int rows = train_blocks(n);
+    hipLaunchKernelGGL(k_train_tile, dim3(rows), dim3(64 * kTrainWaves), 0, c->stream, c->x, c->t, n, c->p, c->wb,
+                       c->part);
+    hipLaunchKernelGGL(k_sum_and_step, dim3((kPart + kBlock / kSumWays - 1) / (kBlock / kSumWays)), dim3(kBlock), 0,
+                       c->stream, c->part, rows, n, c->g, c->loss, c->p, c->m, c->v, c->wb, lr, c1, c2);
 }
 
 int upload(dem_closure* c, int64_t n, const float* x, const float* t)
@@ -407,11 +657,17 @@ int dem_closure_create(dem_closure** out, int32_t device)
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc(&c->p, sizeof(float) * kP) != hipSuccess || hipMalloc(&c->m, sizeof(float) * kP) != hipSuccess ||
         hipMalloc(&c->v, sizeof(float) * kP) != hipSuccess || hipMalloc(&c->g, sizeof(float) * kP) != hipSuccess ||
-        hipMalloc(&c->wb, sizeof(uint16_t) * kP) != hipSuccess || hipMemset(c->p, 0, sizeof(float) * kP) != hipSuccess ||
+        hipMalloc(&c->wb, sizeof(uint16_t) * kPacked) != hipSuccess ||
+        hipMemset(c->wb, 0, sizeof(uint16_t) * kPacked) != hipSuccess || hipMalloc(&c->loss, sizeof(float)) != hipSuccess ||
+        hipHostMalloc((void**)&c->hx, sizeof(float) * (kIn + kOut) * kSmallCall + 64,
+                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess || hipMemset(c->p, 0, sizeof(float) * kP) != hipSuccess ||
         hipMemset(c->m, 0, sizeof(float) * kP) != hipSuccess || hipMemset(c->v, 0, sizeof(float) * kP) != hipSuccess) {
         dem_closure_destroy(c);
         return DEM_ERR_DEVICE;
     }
+    c->hy = c->hx + kIn * kSmallCall;
+    c->bad = (int*)(c->hy + kOut * kSmallCall);
+    *c->bad = 0;
     *out = c;
     return DEM_OK;
 }
@@ -422,8 +678,9 @@ int dem_closure_destroy(dem_closure* c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_samples(c);
-    for (void* a : {(void*)c->p, (void*)c->m, (void*)c->v, (void*)c->g, (void*)c->wb})
+    for (void* a : {(void*)c->p, (void*)c->m, (void*)c->v, (void*)c->g, (void*)c->wb, (void*)c->part, (void*)c->loss})
         if (a) (void)hipFree(a);
+    if (c->hx) (void)hipHostFree(c->hx);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return DEM_OK;
@@ -436,6 +693,8 @@ int dem_closure_set_params(dem_closure* c, const float* params)
     CCHK(hipMemcpyAsync(c->p, params, sizeof(float) * kP, hipMemcpyHostToDevice, c->stream));
     CCHK(hipMemsetAsync(c->m, 0, sizeof(float) * kP, c->stream));
     CCHK(hipMemsetAsync(c->v, 0, sizeof(float) * kP, c->stream));
+    pack(c);
+    CCHK(hipGetLastError());
     CCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     return DEM_OK;
@@ -454,14 +713,23 @@ int dem_closure_forward(dem_closure* c, int64_t n, const float* x, float* y)
 {
     if (!c || n < 0 || n > (1 << 24) || (n > 0 && (!x || !y))) return DEM_ERR_ARG;
     if (n == 0) return DEM_OK;
-    if (!finite(x, kIn * n)) return DEM_ERR_ARG;
     CCHK(hipSetDevice(c->device));
-    int r = upload(c, n, x, nullptr);
-    if (r) return r;
-    forward(c, (int)n);
+    const bool small = n <= kSmallCall;
+    if (small) {
+        std::memcpy(c->hx, x, sizeof(float) * kIn * n);
+    } else {
+        const int r = upload(c, n, x, nullptr);
+        if (r) return r;
+    }
+    *c->bad = 0;
+    forward(c, (int)n, small ? c->hx : c->x, small ? c->hy : c->y);
     CCHK(hipGetLastError());
-    CCHK(hipMemcpyAsync(y, c->y, sizeof(float) * kOut * n, hipMemcpyDeviceToHost, c->stream));
     CCHK(hipStreamSynchronize(c->stream));
+    if (__atomic_load_n(c->bad, __ATOMIC_ACQUIRE)) return DEM_ERR_ARG;  // an input is not finite
+    if (small)
+        std::memcpy(y, c->hy, sizeof(float) * kOut * n);
+    else
+        CCHK(hipMemcpy(y, c->y, sizeof(float) * kOut * n, hipMemcpyDeviceToHost));
     return DEM_OK;
 }
 
@@ -470,10 +738,10 @@ int dem_closure_gradient(dem_closure* c, int64_t n, const float* x, const float*
     if (!c || n <= 0 || n > (1 << 24) || !x || !target) return DEM_ERR_ARG;
     if (!finite(x, kIn * n) || !finite(target, kOut * n)) return DEM_ERR_ARG;
     CCHK(hipSetDevice(c->device));
-    int r = upload(c, n, x, target);
+    int r = ensure_part(c, n);
+    if (!r) r = upload(c, n, x, target);
     if (r) return r;
-    forward(c, (int)n);
-    backward(c, (int)n);
+    backward(c, (int)n, 0.0f, 1.0f, 1.0f);
     CCHK(hipGetLastError());
     if (grad) CCHK(hipMemcpyAsync(grad, c->g, sizeof(float) * kP, hipMemcpyDeviceToHost, c->stream));
     if (loss) CCHK(hipMemcpyAsync(loss, c->loss, sizeof(float), hipMemcpyDeviceToHost, c->stream));
@@ -488,15 +756,13 @@ int dem_closure_train(dem_closure* c, int64_t n, const float* x, const float* ta
         return DEM_ERR_ARG;
     if (!finite(x, kIn * n) || !finite(target, kOut * n)) return DEM_ERR_ARG;
     CCHK(hipSetDevice(c->device));
-    int r = upload(c, n, x, target);
+    int r = ensure_part(c, n);
+    if (!r) r = upload(c, n, x, target);
     if (r) return r;
     for (int e = 0; e < epochs; ++e) {
-        forward(c, (int)n);
-        backward(c, (int)n);
         ++c->step;
         const float c1 = 1.0f - std::pow(0.9f, (float)c->step), c2 = 1.0f - std::pow(0.999f, (float)c->step);
-        hipLaunchKernelGGL(k_adam, dim3(blocks(kP)), dim3(kBlock), 0, c->stream, c->p, c->m, c->v, c->g, kP, lr, c1,
-                           c2);
+        backward(c, (int)n, lr, c1, c2);
     }
     CCHK(hipGetLastError());
     if (loss) CCHK(hipMemcpyAsync(loss, c->loss, sizeof(float), hipMemcpyDeviceToHost, c->stream));

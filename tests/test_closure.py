@@ -179,6 +179,36 @@ def test_closure128_kernels_against_oracle():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 127, 129, 2048, 2049, 16385])
+def test_closure128_sample_counts_around_the_tiles(n):
+    """Sample counts around the 16 of a wavefront, the 64 and 128 of a block,
+    the largest call through pinned memory (2048), and one that gives the 256
+    training blocks a second tile, against the oracle with the same BF16
+    roundings; a non-finite input is refused and leaves the output alone."""
+    x, t = samples(n, 6)
+    net = closure.Closure(seed=9)
+    p = net.params()
+    y, yo = net(x), O.forward128(p, x)[0]
+    scale = np.abs(yo).max()
+    err = np.abs(y - yo)
+    # an activation that rounds the other way moves by 2^-8 of itself, and an
+    # output, a sum of such terms none of which exceeds its scale, by at most
+    # 2^-8 of the scale (seldom: see above; all but a few agree to FP32 rounding)
+    assert err.max() <= 2.0 ** -8 * scale, err.max() / scale
+    assert np.sum(err > 1e-5 * scale) <= max(2, 0.01 * err.size)
+    loss, g = net.gradient(x, t)
+    lo, go = O.loss_and_gradient128(p, x, t)
+    # the outputs' error in the squares
+    assert abs(loss - lo) <= 2.0 ** -7 * scale * np.sqrt(2.0 * lo) + 2.0 ** -15 * scale ** 2
+    np.testing.assert_allclose(g, go, rtol=0, atol=1e-3 * np.abs(go).max())
+    bad = x.copy()
+    bad[n // 2, 1] = np.inf
+    with pytest.raises(RuntimeError):
+        net(bad)
+    np.testing.assert_array_equal(net(x), y)
+
+
+@pytest.mark.gpu
 def test_closure128_trained_beats_constant():
     xtr, ttr = samples(4000, 3)
     xte, tte = samples(1000, 4)

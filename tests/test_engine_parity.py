@@ -1014,7 +1014,7 @@ def test_batches_of_steps_equal_single_steps(skin):
     takes back those that found their lists outdated: every n around the
     batch sizes gives what n calls of dem_step(1) give, bit for bit, with the
     same number of rebuilds and clock, and profiled as well."""
-    sc = S.mixture(n=200, seed=93, lx=5.0, ly=5.0, lz=5.0, inflate=1.08, vmax=3.0, laws="hvm",
+    sc = S.mixture(n=200, seed=93, lx=6.0, ly=6.0, lz=6.0, inflate=1.08, vmax=3.0, laws="hvm",
                    periodic=(True, False), walls=("bottom", "top"))
     engines = [dem.Engine(skin=skin) for _ in range(3)]
     for e in engines:
