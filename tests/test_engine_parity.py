@@ -1038,3 +1038,19 @@ def test_batches_of_steps_equal_single_steps(skin):
     assert s.n_rebuilds > 3
     assert profiled.stats().n_timed_steps == total
     assert_contacts_equal(batched, single)
+
+
+@pytest.mark.parametrize("points", [1, 7, 64, 1001])
+def test_cg_chunks_of_particles(points):
+    """Points for which a thread's chunk of particles is the smallest, a part
+    of the last chunk, and longer (5 particles): the oracle's fields, whose
+    sums run over all particles in order, within rounding."""
+    sc = S.mixture(n=601, seed=94, lx=8.0, ly=8.0, lz=8.0, inflate=1.1, laws="hvm", periodic=(True, True),
+                   walls=("bottom",))
+    g, o = make_pair(sc)
+    for e in (g, o):
+        e.compute_forces()
+    a, b = (e.cg_z(points, 0.6, (0.0, 0.0, 0.0), (8.0, 8.0, 8.5)) for e in (g, o))
+    scale = np.abs(b).max(axis=0)
+    # (the bar of test_engine_cg_vs_oracle)
+    assert np.all(np.abs(a - b) <= 1e-10 * scale), np.max(np.abs(a - b) / np.maximum(scale, 1e-300))
