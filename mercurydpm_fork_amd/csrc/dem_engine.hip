@@ -87,8 +87,12 @@ enum Flag {
     F_DONE_BLOCKS = 12, // blocks of the last rebuild kernel that have finished
     F_NONFINITE = 13,   // a particle position is not finite: the run diverged
     F_STEP = 14,        // the step counter of steps replayed from a captured graph
-    F_PRUNE_AT = 15,    // number of the force pass that has to prune the lists (step_pass)
-    F_NUM = 16
+    // number of the even (0) and odd (1) force pass that has to prune the lists
+    // (step_pass): while a pass's late blocks still read its own word, its early
+    // blocks may already ask for the next pass
+    F_PRUNE_AT0 = 15,
+    F_PRUNE_AT1 = 16,
+    F_NUM = 17
 };
 
 // Integration fused into the force kernel: none (a force pass only), the
@@ -389,7 +393,7 @@ __device__ inline void ask_lists(const Params& p, int* flags, int needs, uint32_
             __atomic_store_n(p.rebuild_word, (uint32_t)at, __ATOMIC_RELAXED);
         }
     }
-    if (needs & NEEDS_PRUNE) __atomic_store_n(&flags[F_PRUNE_AT], (int)pass, __ATOMIC_RELAXED);
+    if (needs & NEEDS_PRUNE) __atomic_store_n(&flags[F_PRUNE_AT0 + (pass & 1)], (int)pass, __ATOMIC_RELAXED);
 }
 
 // floor(v) as a cell coordinate, clamped to +-2^29 (NaN: 0), so that cell
@@ -1143,7 +1147,7 @@ __global__ void __launch_bounds__(kBlock) k_orphans(Dev<NS> d, Params p)
             d.flags[F_DONE_BLOCKS] = 0;
             d.flags[F_REBUILD] = 0;
             d.flags[F_REBUILDS] += 1;
-            d.flags[F_PRUNE_AT] = (int)step_pass(p);
+            d.flags[F_PRUNE_AT0 + (step_pass(p) & 1)] = (int)step_pass(p);
             d.flags[F_ORPH_COUNT0 + (par ^ 1)] = 0;
             d.flags[F_ORPH_PARITY] = par;
         }
@@ -1196,8 +1200,8 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 // entries within the sum of the radii plus a smaller skin (Params::inner), in
 // list order; the passes that follow walk those (about 3 per particle), which
 // holds until some particle has moved half the smaller skin: integrate() then
-// asks the next pass to prune (F_PRUNE_AT carries that pass's number, so a pass
-// and the one that asks never race).  Every contact is found, in the same
+// asks the next pass to prune (a word for even and one for odd passes, with the
+// pass's number: a pass and the requests made in it never meet).  Every contact is found, in the same
 // order, so the results are bit-identical.
 //
 // What bounds it (2M chute, 0.2 to 0.9 contacts per particle): the state alone,
@@ -1468,7 +1472,7 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     // the wavefront's packed lists are walked as one flat sequence of `total`
     // entries starting at wbase * stride: the pruned ones, or all of them in a
     // pass that prunes
-    const bool prune = (uint32_t)__atomic_load_n(&d.flags[F_PRUNE_AT], __ATOMIC_RELAXED) == pass;
+    const bool prune = (uint32_t)__atomic_load_n(&d.flags[F_PRUNE_AT0 + (pass & 1)], __ATOMIC_RELAXED) == pass;
     const uint2* __restrict__ list = prune ? d.nbrc : d.nbri;
     const int total = __builtin_amdgcn_readfirstlane((int)(prune ? d.gtot : d.itot)[wave]);
     const size_t lbase = (size_t)wbase * p.maxn;
