@@ -1082,3 +1082,40 @@ def test_prune_requests_in_consecutive_passes():
         for k in a:
             np.testing.assert_array_equal(a[k], b[k], err_msg=k)
         np.testing.assert_array_equal(ca.spring, cb.spring)
+
+
+@pytest.mark.parametrize("n", [1, 255, 8192, 8193])
+def test_state_read_and_set_through_either_staging(n):
+    """Sizes around the largest system whose state goes through pinned
+    memory: the state comes back in handler order as it was sent (ids out of
+    order in space, some particles removed before), any array may be left
+    out, and dem_set_kinematics sets what it is given."""
+    sc = S.chute_hvm(n_flow=9000, seed=6, l=24.4, depth=10.0)
+    pick = np.random.default_rng(n).permutation(sc.state.n)[:n + 40]
+    sc = _subset(sc, np.sort(pick))
+    rng = np.random.default_rng(4)
+    sc.state.w[:] = rng.normal(0.0, 1.0, sc.state.w.shape)
+    sc.state.q[:] = rng.normal(0.0, 1.0, sc.state.q.shape)
+    f, t = rng.normal(0.0, 1.0, (2, n + 40, 3))
+    sc.state.f, sc.state.t = f, t
+    e = dem.Engine()
+    S.apply(e, sc)
+    order = np.arange(n + 40)
+    for k in range(40):  # removeObject: the last particle takes the index
+        i = (7 * k) % (n + 40 - k)
+        e.remove_particles([i])
+        order[i] = order[n + 39 - k]
+        order = order[:n + 39 - k]
+    want = dict(x=sc.state.x, v=sc.state.v, w=sc.state.w, q=sc.state.q, f=f, t=t)
+    got = e.download()
+    for k in want:
+        np.testing.assert_array_equal(got[k], want[k][order], err_msg=k)
+    v, q = rng.normal(0.0, 1.0, (n, 3)), rng.normal(0.0, 1.0, (n, 4))
+    e.set_kinematics(v=v, q=q)
+    got = e.download()
+    np.testing.assert_array_equal(got["v"], v)
+    np.testing.assert_array_equal(got["q"], q)
+    np.testing.assert_array_equal(got["x"], sc.state.x[order])
+    only = np.full((n, 3), np.nan)
+    e._check(e.lib.dem_download_particles(e.h, None, None, dem._ptr(only), None, None, None))
+    np.testing.assert_array_equal(only, sc.state.w[order])
