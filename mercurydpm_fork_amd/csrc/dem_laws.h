@@ -29,7 +29,7 @@ struct ContactGeom {
 
 // Force laws a kernel can be specialised for when every species pair uses
 // them (the operations are the same as on the general path).
-enum { LAW_ANY = 0, LAW_HERTZ_MINDLIN = 1 };
+enum { LAW_ANY = 0, LAW_HERTZ_MINDLIN = 1, LAW_LINEAR_FRICTION = 2 };  // (2: linear normal law, FULL friction)
 
 // Returns the contact force on P, the contact torque (the part added with
 // addTorque; the lever-arm torque is applied by the caller) and the
@@ -50,7 +50,7 @@ __device__ inline void contact_force(const dem_pair_params& s, const Body& P, co
     const double eff_m = 1.0 / (P.inv_mass + (g.i_is_wall ? 0.0 : I.inv_mass));
     if (g.overlap > 0) {
         double fn;
-        if (LAW != LAW_HERTZ_MINDLIN && s.normal_law == DEM_NORMAL_LINEAR_VISCOELASTIC) {
+        if (LAW == LAW_LINEAR_FRICTION || (LAW == LAW_ANY && s.normal_law == DEM_NORMAL_LINEAR_VISCOELASTIC)) {
             fn = s.stiffness * g.overlap - s.dissipation * nrv;
             if (s.constant_restitution) fn *= 2.0 * eff_m;
         } else {
@@ -68,7 +68,7 @@ __device__ inline void contact_force(const dem_pair_params& s, const Body& P, co
     }
     if (fn_abs == 0.0) return;
 
-    if (LAW == LAW_HERTZ_MINDLIN || s.friction_law == DEM_FRICTION_MINDLIN) {
+    if (LAW == LAW_HERTZ_MINDLIN || (LAW == LAW_ANY && s.friction_law == DEM_FRICTION_MINDLIN)) {
         if (s.sliding_mu != 0.0) {
             const V3 vt = vsub(rel_vel, vmul(g.normal, nrv));
             V3 xi = mk(spring[0], spring[1], spring[2]);
@@ -98,7 +98,7 @@ __device__ inline void contact_force(const dem_pair_params& s, const Body& P, co
         }
         return;
     }
-    if (s.friction_law == DEM_FRICTION_NONE) return;
+    if (LAW == LAW_ANY && s.friction_law == DEM_FRICTION_NONE) return;
 
     // --- sliding friction (SLIDING and FULL)
     if (s.sliding_mu != 0.0) {
@@ -141,7 +141,7 @@ __device__ inline void contact_force(const dem_pair_params& s, const Body& P, co
         }
     }
     if constexpr (NS == 9) {
-        if (s.friction_law != DEM_FRICTION_FULL) return;
+        if (LAW == LAW_ANY && s.friction_law != DEM_FRICTION_FULL) return;
         if (s.rolling_mu != 0.0 && s.rolling_stiffness != 0.0) {
             const double eff_d = 2.0 * eff_r;
             const V3 rrv = vmul(vcross(g.normal, vsub(P.omega, I.omega)), -eff_d);

@@ -89,7 +89,7 @@ __device__ inline void contact_force_mixed(const dem_pair_params& s, double rP, 
     const float eff_m = 1.0f / (float)(invP + (g.i_is_wall ? 0.0 : invI));
     if (!(g.overlap > 0.f)) return;
     float fn;
-    if (LAW != LAW_HERTZ_MINDLIN && s.normal_law == DEM_NORMAL_LINEAR_VISCOELASTIC) {
+    if (LAW == LAW_LINEAR_FRICTION || (LAW == LAW_ANY && s.normal_law == DEM_NORMAL_LINEAR_VISCOELASTIC)) {
         fn = (float)s.stiffness * g.overlap - (float)s.dissipation * nrv;
         if (s.constant_restitution) fn *= 2.0f * eff_m;
     } else {
@@ -102,7 +102,7 @@ __device__ inline void contact_force_mixed(const dem_pair_params& s, double rP, 
     if (fn_abs == 0.f) return;
     const V3 nd = fd(g.normal);
 
-    if (LAW == LAW_HERTZ_MINDLIN || s.friction_law == DEM_FRICTION_MINDLIN) {
+    if (LAW == LAW_HERTZ_MINDLIN || (LAW == LAW_ANY && s.friction_law == DEM_FRICTION_MINDLIN)) {
         if (s.sliding_mu != 0.0) {
             const F3 vt = fsub(g.vrel, fmul(g.normal, nrv));
             V3 xi = mk(spring[0], spring[1], spring[2]);
@@ -132,7 +132,7 @@ __device__ inline void contact_force_mixed(const dem_pair_params& s, double rP, 
         }
         return;
     }
-    if (s.friction_law == DEM_FRICTION_NONE) return;
+    if (LAW == LAW_ANY && s.friction_law == DEM_FRICTION_NONE) return;
 
     if (s.sliding_mu != 0.0) {
         const F3 vt = fsub(g.vrel, fmul(g.normal, nrv));
@@ -171,7 +171,7 @@ __device__ inline void contact_force_mixed(const dem_pair_params& s, double rP, 
         }
     }
     if constexpr (NS == 9) {
-        if (s.friction_law != DEM_FRICTION_FULL) return;
+        if (LAW == LAW_ANY && s.friction_law != DEM_FRICTION_FULL) return;
         const float eff_d = 2.0f * eff_r;
         const F3 dw = ff(vsub(wPd, wId));
         if (s.rolling_mu != 0.0 && s.rolling_stiffness != 0.0) {

@@ -1119,3 +1119,32 @@ def test_state_read_and_set_through_either_staging(n):
     only = np.full((n, 3), np.nan)
     e._check(e.lib.dem_download_particles(e.h, None, None, dem._ptr(only), None, None, None))
     np.testing.assert_array_equal(only, sc.state.w[order])
+
+
+@pytest.mark.parametrize("laws", ["full", "box"])
+@pytest.mark.parametrize("precision", [dem.PRECISION_FP64, dem.PRECISION_MIXED], ids=["fp64", "mixed"])
+def test_linear_friction_kernel_equals_the_general_one(laws, precision):
+    """The force kernel specialised for linear laws with full friction (with
+    and without rolling) against the general one: the general kernel is
+    taken when a further species pair, which no particle belongs to, has
+    another law.  Bit-identical."""
+    if laws == "full":
+        sc = S.mixture(n=300, seed=95, lx=6.0, ly=6.0, lz=6.0, inflate=1.1, laws="full", periodic=(True, True),
+                       walls=("bottom", "top"))
+    else:
+        sc = S.box_lvf(n=600, lx=8.0, ly=8.0, lz=16.0)
+        sc.state.radius[:] *= 1.04
+    general = S.Scenario(sc.name, list(sc.species) + [S.Species(density=1.0)], sc.walls, sc.periodic, sc.gravity, sc.dt,
+                         sc.state, rotation=sc.uses_rotation())
+    outs = []
+    for k in (sc, general):
+        e = dem.Engine(precision=precision)
+        S.apply(e, k)
+        e.compute_forces()
+        e.step(40)
+        outs.append((e.download(), e.contacts()))
+    (a, ca), (b, cb) = outs
+    assert ca.n > 20
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+    np.testing.assert_array_equal(ca.spring, cb.spring)
