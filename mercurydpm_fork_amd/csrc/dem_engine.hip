@@ -160,7 +160,6 @@ struct Dev {
     // Verlet lists
     uint32_t* nbr;
     int32_t* ncount;
-    uint8_t* rev;
     // the same lists packed back to back per wavefront of g = Params::group
     // particles: the lists of particles gw .. gw+g-1 fill, in order, the
     // region starting at gw * stride -- what the force kernel walks, gtot[w]
@@ -1106,30 +1105,61 @@ __global__ void __launch_bounds__(kBlock) k_rematch(Dev<NS> d, Params p, int cur
         if (!valid) continue;
         const uint32_t idi = d.t_id[i];
         unsigned long long m = 0;
-        for (int k = 0; k < cnt; ++k) {
-            const size_t sl = lslot(k, p.maxn, i);
-            const uint32_t e = d.nbr[sl];
-            const uint32_t j = e & ~kWriterBit;
-            const uint32_t at = (uint32_t)k << 8 | (uint32_t)at_group << 14;
-            if (e & kWriterBit) {
-                Rec<NS> r;
-                if (hash_find(d, ((uint64_t)idi << 32) | d.t_id[j], r)) {
-                    d.rec[cur][sl] = r;
-                    m |= 1ull << k;
-                }
-                d.rev[sl] = 0xFF;
-                d.nbrc[off + k] = make_uint2(e, at | 0xFFu);
-            } else {
-                const int cj = d.ncount[j];
-                int kk = -1;
-                for (int a = 0; a < cj; ++a)
-                    if ((d.nbr[lslot(a, p.maxn, (int)j)] & ~kWriterBit) == (uint32_t)i) {
-                        kk = a;
-                        break;
+        // kAhead entries at a time: their partners, then what each first needs of
+        // its partner (a writer the first hash slot of the pair, a reader the
+        // length and the first entries of the partner's list), are loaded
+        // together: a thread's chain of dependent loads bounds the kernel (one
+        // entry at a time 153 us at 211,000 spheres and 1.7 ms at 2.08M, so 117
+        // us and 1.24 ms)
+        constexpr int kAhead = 4;
+        for (int k0 = 0; k0 < cnt; k0 += kAhead) {
+            uint32_t e[kAhead], found[kAhead];
+            uint64_t key[kAhead], h[kAhead];
+            unsigned long long first[kAhead];
+            int cj[kAhead];
+            uint32_t head[kAhead][kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) e[u] = d.nbr[lslot(min(k0 + u, cnt - 1), p.maxn, i)];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const uint32_t j = e[u] & ~kWriterBit;
+                key[u] = ((uint64_t)idi << 32) | d.t_id[j];
+                cj[u] = d.ncount[j];
+#pragma unroll
+                for (int a = 0; a < kAhead; ++a) head[u][a] = d.nbr[lslot(min(a, p.maxn - 1), p.maxn, (int)j)];
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                h[u] = mix64(key[u]) & (d.hcap - 1);
+                first[u] = (e[u] & kWriterBit) ? d.hkey[h[u]] : kEmptyKey;
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int k = k0 + u;
+                if (k >= cnt) break;
+                const size_t sl = lslot(k, p.maxn, i);
+                const uint32_t at = (uint32_t)k << 8 | (uint32_t)at_group << 14;
+                found[u] = 0xFFu;
+                if (e[u] & kWriterBit) {
+                    Rec<NS> r;
+                    if (first[u] != kEmptyKey && hash_find(d, key[u], r)) {
+                        d.rec[cur][sl] = r;
+                        m |= 1ull << k;
                     }
-                if (kk < 0) atomicOr(&d.flags[F_LIST_ASYM], 1);
-                d.rev[sl] = (uint8_t)(kk < 0 ? 0xFF : kk);
-                d.nbrc[off + k] = make_uint2(e, at | (kk < 0 ? 0xFFu : (uint32_t)kk));
+                } else {
+                    const uint32_t j = e[u] & ~kWriterBit;
+                    int kk = -1;
+#pragma unroll
+                    for (int a = kAhead - 1; a >= 0; --a)
+                        if (a < cj[u] && (head[u][a] & ~kWriterBit) == (uint32_t)i) kk = a;
+                    for (int a = kAhead; kk < 0 && a < cj[u]; ++a)
+                        if ((d.nbr[lslot(a, p.maxn, (int)j)] & ~kWriterBit) == (uint32_t)i) kk = a;
+                    if (kk < 0)
+                        atomicOr(&d.flags[F_LIST_ASYM], 1);
+                    else
+                        found[u] = (uint32_t)kk;
+                }
+                d.nbrc[off + k] = make_uint2(e[u], at | found[u]);
             }
         }
         d.mask[cur][i] = m;
@@ -2891,7 +2921,7 @@ int alloc_particles(dem_ctx* ctx, int64_t n)
     A(d.t_id, n) A(d.t_orig, n) A(d.t_spc, n) A(d.t_cellc, n);
     const size_t slots = (size_t)n * ctx->maxn_cfg;
     const size_t wslots_packed = ((size_t)n + 63) / 64 * 64 * ctx->maxn_cfg;
-    A(d.nbr, slots) A(d.ncount, n) A(d.rev, slots) A(d.nbrc, wslots_packed) A(d.nbri, wslots_packed);
+    A(d.nbr, slots) A(d.ncount, n) A(d.nbrc, wslots_packed) A(d.nbri, wslots_packed);
     const size_t waves = ((size_t)n + ctx->prm.group - 1) / ctx->prm.group;
     A(d.gtot, waves) A(d.itot, waves);
     A(d.rec[0], slots) A(d.rec[1], slots) A(d.mask[0], n) A(d.mask[1], n) A(d.fc, slots) A(d.ftc, slots);
