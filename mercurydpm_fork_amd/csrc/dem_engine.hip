@@ -372,6 +372,12 @@ __device__ inline bool prune_due(const Params& p, double4 ds)
     return !(dx * dx + dy * dy + dz * dz <= p.inner_thr2);
 }
 
+// A flag word as it was when the kernel started, or later.
+__device__ inline int load_flag(const int* flags, int word)
+{
+    return __hip_atomic_load(&flags[word], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // The rebuild flag: the number of the first force pass that must not run on
 // the present lists, doubled, plus one (so that it is never 0).
 __host__ __device__ inline uint32_t rebuild_at(uint32_t pass) { return pass << 1 | 1u; }
@@ -1292,8 +1298,8 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 // read and written with the integration, takes 163 us (770 MB, 4.7 TB/s, the
 // rate of a large copy); walking the pruned lists adds about 80 us and the
 // contacts 70 to 190, waiting for gathers.  437 us per pass with pruning and
-// with the sums taken lane to lane (16 KB less LDS per block), 462 before.
-// Four wavefronts per SIMD (128 registers, spilling) took 491, two lanes
+// with the sums taken lane to lane (16 KB less LDS per block), 462 before; 424
+// since a pass loads all it starts from at once.  Four wavefronts per SIMD (128 registers, spilling) took 491, two lanes
 // loading each record together 441.
 
 // v of lane src
@@ -1507,12 +1513,27 @@ __device__ inline void process_batch(Dev<NS>& d, const Params& p, int cur, Owner
 template <int NS, int LAW, int PREC>
 __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Params p, int cur)
 {
-    // a diverged state (non-finite position, found by the rebuild) gets no
-    // force pass: its lists were not rebuilt; neither does one that needs new
-    // lists (the host rebuilds them and launches the pass again: run_passes)
-    if (__atomic_load_n(&d.flags[F_NONFINITE], __ATOMIC_RELAXED)) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = xcd_block() * kWaves + (int)(threadIdx.x >> 6);
+    const int wbase = wave * p.group;  // the wavefront's particles are wbase .. wbase + p.group - 1
+    const int i = wbase + lane;
+    const bool valid = lane < p.group && i < p.n;
     const uint32_t pass = step_pass(p);
-    if (waits_for_rebuild((uint32_t)__atomic_load_n(&d.flags[F_REBUILD], __ATOMIC_RELAXED), pass)) return;
+    // Everything that the pass starts from is loaded at once: the flag words,
+    // the owners' state and the lengths of both packed lists.  (The flags change
+    // during the pass only in ways it must not see, or need not: a cached load
+    // will do.  2M chute: 436 us per pass with the flags read one after another
+    // past the caches and the rest after them, 424 so.)
+    const int nonfinite = load_flag(d.flags, F_NONFINITE);
+    const uint32_t rebuild = (uint32_t)load_flag(d.flags, F_REBUILD);
+    const uint32_t prune_at = (uint32_t)load_flag(d.flags, F_PRUNE_AT0 + (int)(pass & 1));
+    const int ii = valid ? i : 0;
+    const int w0 = wbase < p.n ? wave : 0;
+    const uint32_t total_all = d.gtot[w0], total_pruned = d.itot[w0];
+    const double4 pr0 = d.posr[ii];
+    const double4 vl0 = d.vel[ii];
+    const double4 om0 = d.omg[ii];
+    const uint32_t spc0 = d.spc[ii];
     __shared__ OwnerLds lds[kWaves];
     __shared__ LawLds law;
     if constexpr (LAW == LAW_HERTZ_MINDLIN) {
@@ -1528,39 +1549,31 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
         }
         __syncthreads();
     }
-    const int lane = threadIdx.x & 63;
+    // a diverged state (non-finite position, found by the rebuild) gets no
+    // force pass: its lists were not rebuilt; neither does one that needs new
+    // lists (the host rebuilds them and launches the pass again: run_passes)
+    if (nonfinite || waits_for_rebuild(rebuild, pass) || wbase >= p.n) return;
     OwnerLds& L = lds[threadIdx.x >> 6];
-    const int wave = xcd_block() * kWaves + (int)(threadIdx.x >> 6);
-    const int wbase = wave * p.group;  // the wavefront's particles are wbase .. wbase + p.group - 1
-    if (wbase >= p.n) return;
-    const int i = wbase + lane;
-    const bool valid = lane < p.group && i < p.n;
-    const int ii = valid ? i : wbase;
-    {
-        // the owners' state goes to LDS for the contact phase; the epilogue
-        // reads it back, so that it occupies no registers meanwhile
-        const double4 pr = d.posr[ii];
-        const double4 vl = d.vel[ii];
-        const double4 om = d.omg[ii];
-        L.px[lane] = pr.x;
-        L.py[lane] = pr.y;
-        L.pz[lane] = pr.z;
-        L.r[lane] = pr.w;
-        L.vx[lane] = vl.x;
-        L.vy[lane] = vl.y;
-        L.vz[lane] = vl.z;
-        L.im[lane] = vl.w;
-        L.wx[lane] = om.x;
-        L.wy[lane] = om.y;
-        L.wz[lane] = om.z;
-        L.sp[lane] = (int)(d.spc[ii] & 0xFFFF);
-    }
+    // the owners' state goes to LDS for the contact phase; the epilogue reads
+    // it back, so that it occupies no registers meanwhile
+    L.px[lane] = pr0.x;
+    L.py[lane] = pr0.y;
+    L.pz[lane] = pr0.z;
+    L.r[lane] = pr0.w;
+    L.vx[lane] = vl0.x;
+    L.vy[lane] = vl0.y;
+    L.vz[lane] = vl0.z;
+    L.im[lane] = vl0.w;
+    L.wx[lane] = om0.x;
+    L.wy[lane] = om0.y;
+    L.wz[lane] = om0.z;
+    L.sp[lane] = (int)(spc0 & 0xFFFF);
     // the wavefront's packed lists are walked as one flat sequence of `total`
     // entries starting at wbase * stride: the pruned ones, or all of them in a
     // pass that prunes
-    const bool prune = (uint32_t)__atomic_load_n(&d.flags[F_PRUNE_AT0 + (pass & 1)], __ATOMIC_RELAXED) == pass;
+    const bool prune = prune_at == pass;
     const uint2* __restrict__ list = prune ? d.nbrc : d.nbri;
-    const int total = __builtin_amdgcn_readfirstlane((int)(prune ? d.gtot : d.itot)[wave]);
+    const int total = __builtin_amdgcn_readfirstlane((int)(prune ? total_all : total_pruned));
     const size_t lbase = (size_t)wbase * p.maxn;
     uint32_t kept = 0;
     unsigned long long touched = 0;
@@ -3223,13 +3236,22 @@ void rebuild_now(dem_ctx* ctx, int erase)
 // takes back the passes that did nothing, rebuilds and goes on.  (Nine rebuild
 // kernels per step that return at once cost 17 to 25 us per step: more than
 // the force pass of a few thousand spheres.)  Batches are an eighth of the
-// passes between rebuilds, 4 to 16: a rebuild then wastes about one and a half
-// batches of passes that return at once (2 to 3 us each) and one wait.
+// passes between rebuilds, 4 to 16 (4 above kLongPass particles, whose passes
+// are long enough to launch the next batch under): a rebuild then wastes about
+// one and a half batches of passes that do nothing but load their first data (2
+// to 3 us each, 40 us at 2M) and one wait.
+constexpr int64_t kLongPass = 500000;
+constexpr int kMaxBatch = 16;
+int batch_of(const dem_ctx* ctx)
+{
+    if (ctx->n > kLongPass) return 4;
+    return (int)std::min<int64_t>(kMaxBatch, std::max<int64_t>(4, ctx->since_rebuild / 8));
+}
+
 template <int NS>
 int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
 {
     const bool prof = ctx->profiling;
-    constexpr int kMaxBatch = 16;
     // profiling: two events per pass in flight, two for the rebuild
     if (prof) {
         const int r = ensure_events(ctx, 4 * kMaxBatch + 2);
@@ -3265,6 +3287,7 @@ int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
         for (int64_t s = done; s < upto && steps; ++s) advance_clock(ctx);
         ctx->since_rebuild += upto - done;
         done = upto;
+        ctx->batch = std::max(ctx->batch, batch_of(ctx));
         return DEM_OK;
     };
     while (done < n) {
@@ -3304,7 +3327,7 @@ int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
         if ((r = finish(sent)) != 0) return r;
         flying = 0;
         if (flag) {
-            ctx->batch = (int)std::min<int64_t>(kMaxBatch, std::max<int64_t>(4, ctx->since_rebuild / 8));
+            ctx->batch = batch_of(ctx);
             *ctx->rebuild_word = 0;
             if ((r = rebuild()) != 0) return r;
         }
