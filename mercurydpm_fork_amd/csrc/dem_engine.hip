@@ -14,8 +14,9 @@
 // a bucket, and a Verlet list (radius sum + skin, minimum image across periodic
 // boundaries) is built from the sorted cells.  The list is rebuilt when any
 // particle has moved more than half the skin; the decision is taken on the
-// device (the rebuild kernels exit at once when no rebuild is flagged), so a
-// dem_step() call never synchronises with the host until it returns.
+// device: a force pass that finds its lists outdated does nothing, and the host,
+// which launches passes ahead in batches, rebuilds and goes on (run_passes).
+// Between rebuilds the force passes walk pruned lists of a smaller skin.
 // Contact history: one record per stored interaction, in the list slot of its
 // writer (the lower id), double-buffered across steps.  On every rebuild the
 // active records go into a device hash table keyed by (id_lo, id_hi) or
@@ -1267,14 +1268,16 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 // this pass are dropped when their time stamp is not newer than the step
 // counter (eraseOldInteractions, InteractionHandler.cc:377-393).
 // ------------------------------------------------------------------------
-// The kernel works per wavefront of 64 particles ("owners", one per lane):
-//  scan   -- every lane walks its Verlet list and tests the contact
-//            predicate; contacts are compacted into an LDS queue with a
-//            wavefront ballot + prefix count (mbcnt), so
+// The kernel works per wavefront of Params::group particles ("owners", one per
+// lane):
+//  scan   -- the wavefront walks its owners' packed lists, 64 entries at a time,
+//            and tests the contact predicate; contacts are compacted into an
+//            LDS queue with a wavefront ballot + prefix count (mbcnt), so
 //  process -- the force law runs with all 64 lanes busy, one queued contact
 //            each, instead of diverging over list entries that are not in
-//            contact.  Contributions go to LDS and each owner adds its own in
-//            queue order, i.e. in list order: the sum is deterministic.
+//            contact.  Each owner then reads its contributions out of the
+//            lanes that evaluated them, in queue order, i.e. in list order: the
+//            sum is deterministic.
 // Both particles of a pair evaluate it (no atomics); the lower id writes the
 // history record.
 // A packed list entry names its owner and its slot in the owner's list: finding
