@@ -390,18 +390,28 @@ __host__ __device__ inline bool waits_for_rebuild(uint32_t flag, uint32_t pass)
     return flag != 0 && (int32_t)(flag - rebuild_at(pass)) <= 0;
 }
 
-// What integrate() asks of the list upkeep, for the force pass `pass`.
+// What integrate() asks of the list upkeep, for the force pass `pass`.  One
+// lane asks for its wavefront, and only while the word does not hold the
+// request yet: particles that move together cross the skin in the same pass,
+// and their stores to the one word wait for each other (2.0M spheres of one
+// speed, no contacts: a pass after which none asks takes 0.137 ms; one after
+// which all ask took 1.31 ms with a store per lane, and takes 0.18 ms so).
 enum { NEEDS_REBUILD = 1, NEEDS_PRUNE = 2 };
+__device__ inline bool write_request(int* word, int value)
+{
+    if (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == value) return false;
+    __hip_atomic_store(word, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
 __device__ inline void ask_lists(const Params& p, int* flags, int needs, uint32_t pass)
 {
-    if (needs & NEEDS_REBUILD) {
+    const unsigned long long rebuild = __ballot(needs & NEEDS_REBUILD), prune = __ballot(needs & NEEDS_PRUNE);
+    const int lane = threadIdx.x & 63;
+    if (rebuild && lane == __ffsll((long long)rebuild) - 1) {
         const int at = (int)rebuild_at(pass);
-        if (__atomic_load_n(&flags[F_REBUILD], __ATOMIC_RELAXED) != at) {
-            __atomic_store_n(&flags[F_REBUILD], at, __ATOMIC_RELAXED);
-            __atomic_store_n(p.rebuild_word, (uint32_t)at, __ATOMIC_RELAXED);
-        }
+        if (write_request(&flags[F_REBUILD], at)) __atomic_store_n(p.rebuild_word, (uint32_t)at, __ATOMIC_RELAXED);
     }
-    if (needs & NEEDS_PRUNE) __atomic_store_n(&flags[F_PRUNE_AT0 + (pass & 1)], (int)pass, __ATOMIC_RELAXED);
+    if (prune && lane == __ffsll((long long)prune) - 1) write_request(&flags[F_PRUNE_AT0 + (pass & 1)], (int)pass);
 }
 
 // floor(v) as a cell coordinate, clamped to +-2^29 (NaN: 0), so that cell

@@ -1183,3 +1183,29 @@ def test_lists_where_cells_share_buckets(kind, sweep):
             e.step_end()
         # (the drift used forces summed in another order: springs to round-off)
         assert assert_contacts_close(g, o) > 50
+
+
+@pytest.mark.parametrize("who", ["all", "one", "two"])
+def test_list_requests_of_any_lane(who):
+    """One lane asks for its wavefront's pruned lists and rebuilds: all
+    spheres crossing the skins in the same passes, one of them (each place in
+    the wavefront in turn) and a pair in different wavefronts, at the sizes of
+    the pruned and of the Verlet skin; the contacts of the oracle, which has
+    no lists."""
+    sc = S.mixture(n=150, seed=96, lx=5.0, ly=5.0, lz=5.0, inflate=1.1, laws="hvm", periodic=(True, True),
+                   walls=("bottom",), vmax=0.01, fixed_frac=0.0)
+    skin = 0.05
+    for k in range(0, 150, 150 if who == "all" else 13):
+        v = sc.state.v.copy()
+        # a fifteenth of the skin per step: the pruned lists last one pass, the Verlet lists seven
+        fast = slice(None) if who == "all" else ([k] if who == "one" else [k, (k + 75) % 150])
+        v[fast] = np.array([0.6, 0.64, 0.48]) * skin / 15.0 / sc.dt
+        g, o = make_pair(sc, skin=skin)
+        for e in (g, o):
+            e.step_begin()
+            e.set_kinematics(v=v)
+            e.step_end()
+            e.step(12)
+        assert g.stats().n_rebuilds >= 2
+        assert assert_contacts_close(g, o) > 0
+        g.close()
