@@ -2764,6 +2764,10 @@ struct dem_ctx {
     hipEvent_t batch_done[2] = {nullptr, nullptr};
     int64_t since_rebuild = 0;        // force passes since the last rebuild of run_passes
     int batch = 8;                    // force passes launched together by run_passes
+    // run_passes: launch the rebuild kernels before every pass; the passes, and
+    // the rebuilds that they asked for, since that was last decided
+    bool rebuild_often = false;
+    int64_t counted_passes = 0, counted_asked = 0;
     int cur = 0;
     Params prm{};
     // device buffers
@@ -3249,16 +3253,37 @@ void rebuild_now(dem_ctx* ctx, int erase)
 // takes back the passes that did nothing, rebuilds and goes on.  (Nine rebuild
 // kernels per step that return at once cost 17 to 25 us per step: more than
 // the force pass of a few thousand spheres.)  Batches are an eighth of the
-// passes between rebuilds, 4 to 16 (4 above kLongPass particles, whose passes
-// are long enough to launch the next batch under): a rebuild then wastes about
+// passes between rebuilds, 4 to 16 (1 to 4 above kLongPass particles, whose
+// passes are long enough to launch the next batch under): a rebuild then wastes about
 // one and a half batches of passes that do nothing but load their first data (2
 // to 3 us each, 40 us at 2M) and one wait.
+//
+// Where a pass in three and a half or more asks, that costs more than the nine
+// kernels before every pass, which need no wait: they are launched so
+// (rebuild_often), up to kMaxOften passes between two looks at how many did ask.
+// A dilute gas that rebuilds every 1, 2, 3, 4 to 5 passes, us per step with
+// batches and so: 2000 spheres 124 / 89, 82 / 66, 58 / 52, 41 / 42; 20,000:
+// 144 / 107, 91 / 75, 63 / 59, 50 / 51; 200,000: 283 / 230, 153 / 137, 109 /
+// 106, 87 / 91; 2.0M: 1626 / 1568, 998 / 985, 563 / 559, 381 / 396 (batches of
+// at least four: 1809, 1119, 604, 415).
+// A call of a pass or two waits for it in any case: a rebuild every 2 passes in
+// calls of one step, 2000 spheres 84 / 102 us per step.
 constexpr int64_t kLongPass = 500000;
-constexpr int kMaxBatch = 16;
+constexpr int kMaxBatch = 16, kMaxOften = 64;
 int batch_of(const dem_ctx* ctx)
 {
-    if (ctx->n > kLongPass) return 4;
-    return (int)std::min<int64_t>(kMaxBatch, std::max<int64_t>(4, ctx->since_rebuild / 8));
+    const bool long_pass = ctx->n > kLongPass;
+    return (int)std::min<int64_t>(long_pass ? 4 : kMaxBatch, std::max<int64_t>(long_pass ? 1 : 4, ctx->since_rebuild / 8));
+}
+
+// Decides rebuild_often from the passes that ran and what they asked for.
+void count_passes(dem_ctx* ctx, int64_t passes, int64_t asked)
+{
+    ctx->counted_passes += passes;
+    ctx->counted_asked += asked;
+    if (ctx->counted_passes < 16) return;
+    ctx->rebuild_often = 7 * ctx->counted_asked >= 2 * ctx->counted_passes;
+    ctx->counted_passes = ctx->counted_asked = 0;
 }
 
 template <int NS>
@@ -3284,7 +3309,11 @@ int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
         return DEM_OK;
     };
     int r;
-    if (ctx->lists_stale && (r = rebuild()) != 0) return r;
+    int expected = ctx->h_flags[F_REBUILDS];  // rebuilds without those still to be asked for
+    if (ctx->lists_stale) {
+        if ((r = rebuild()) != 0) return r;
+        ++expected;
+    }
     int64_t done = 0, sent = 0;  // passes known to have run, passes launched
     int64_t end[2];              // the passes launched when a batch in flight ends
     int oldest = 0, flying = 0;
@@ -3299,11 +3328,28 @@ int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
             }
         for (int64_t s = done; s < upto && steps; ++s) advance_clock(ctx);
         ctx->since_rebuild += upto - done;
+        count_passes(ctx, upto - done, 0);
         done = upto;
         ctx->batch = std::max(ctx->batch, batch_of(ctx));
         return DEM_OK;
     };
     while (done < n) {
+        // (passes are timed one by one when profiling)
+        if (ctx->rebuild_often && !prof && flying == 0 && n - done > 2) {
+            const int64_t first = done, to = std::min(n, done + kMaxOften);
+            for (; done < to; ++done) {
+                rebuild_now<NS>(ctx, erase);
+                launch_force<NS>(ctx, erase, done + 1 < n ? KICK_BOTH : last_kick, (uint32_t)ctx->nt);
+                if (steps) advance_clock(ctx);
+            }
+            HIPCHK(hipGetLastError());
+            sent = done;
+            if ((r = read_flags(ctx)) != 0) return r;
+            count_passes(ctx, done - first, ctx->h_flags[F_REBUILDS] - expected);
+            expected = ctx->h_flags[F_REBUILDS];
+            ctx->batch = batch_of(ctx);
+            continue;
+        }
         while (flying < 2 && sent < n) {
             const int64_t to = std::min(n, sent + ctx->batch);
             for (; sent < to; ++sent) {
@@ -3339,7 +3385,10 @@ int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
         for (int64_t k = 0; k < idle; ++k, --sent) unlaunch_force<NS>(ctx, sent < n ? KICK_BOTH : last_kick);
         if ((r = finish(sent)) != 0) return r;
         flying = 0;
+        expected = ctx->h_flags[F_REBUILDS];
         if (flag) {
+            ++expected;
+            count_passes(ctx, 0, 1);
             ctx->batch = batch_of(ctx);
             *ctx->rebuild_word = 0;
             if ((r = rebuild()) != 0) return r;
@@ -4313,7 +4362,10 @@ static int upload_particles(dem_ctx* ctx, int64_t n, int64_t cap, const uint32_t
     HIPCHK(hipMemcpy(dspc, spc.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
     int flags[F_NUM] = {0};
     flags[F_REBUILD] = (int)rebuild_at(ctx->passes + 1);
+    std::memcpy(ctx->h_flags, flags, sizeof flags);
     ctx->lists_stale = true;
+    ctx->rebuild_often = false;
+    ctx->counted_passes = ctx->counted_asked = 0;
     *ctx->rebuild_word = 0;
     ctx->diverged = false;
     HIPCHK(hipMemcpy(ctx->d_flags, flags, sizeof flags, hipMemcpyHostToDevice));

@@ -1209,3 +1209,45 @@ def test_list_requests_of_any_lane(who):
         assert g.stats().n_rebuilds >= 2
         assert assert_contacts_close(g, o) > 0
         g.close()
+
+
+@pytest.mark.parametrize("every", [1, 2, 4])
+def test_rebuilds_asked_for_in_almost_every_pass(every):
+    """Where a pass in three and a half or more asks for a rebuild, dem_step
+    launches its kernels with every pass; it goes back to batches when they
+    become seldom.  Fast, slow and fast again: bit for bit what calls of one
+    step and a profiled run (which never launch so) give, with the same
+    rebuilds and clock."""
+    sc = S.mixture(n=200, seed=97, lx=6.0, ly=6.0, lz=6.0, inflate=1.05, laws="hvm", periodic=(True, True),
+                   walls=("bottom", "top"), vmax=0.0, fixed_frac=0.0)
+    skin = 0.01
+    rng = np.random.default_rng(2)
+    # all along the floor together, so that they do not run into each other
+    u = np.array([1.0, 0.5, 0.0]) + rng.normal(0.0, 0.01, sc.state.v.shape)
+    u *= 0.5 * skin / (every - 0.5) / sc.dt / np.linalg.norm(u, axis=1)[:, None]
+    engines = [dem.Engine(skin=skin) for _ in range(3)]
+    for e in engines:
+        S.apply(e, sc)
+        e.compute_forces()
+    batched, single, profiled = engines
+    profiled.set_profiling(True)
+    rebuilds = []
+    for speed, steps in ((1.0, 40), (0.02, 150), (1.0, 3), (1.0, 100)):
+        for e in engines:
+            e.step_begin()
+            e.set_kinematics(v=speed * u)
+            e.step_end()
+        before = batched.stats().n_rebuilds
+        batched.step(steps)
+        profiled.step(steps)
+        for _ in range(steps):
+            single.step(1)
+        a, s = batched.download(), batched.stats()
+        rebuilds.append(s.n_rebuilds - before)
+        for e in (single, profiled):
+            b, t = e.download(), e.stats()
+            for k in a:
+                np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+            assert (t.n_steps, t.time, t.n_rebuilds, t.n_contacts) == (s.n_steps, s.time, s.n_rebuilds, s.n_contacts)
+    assert rebuilds[0] >= 40 // (every + 1) and rebuilds[1] < 30 and rebuilds[3] >= 100 // (every + 1)
+    assert_contacts_equal(batched, single)
