@@ -39,6 +39,7 @@
 #include "../../include/mercurydpm_dem.h"
 #include "dem_laws.h"
 #include "dem_laws_mixed.h"
+#include "dem_passes.h"
 #include "dem_vec.h"
 #include "dem_walls.h"
 
@@ -377,17 +378,6 @@ __device__ inline bool prune_due(const Params& p, double4 ds)
 __device__ inline int load_flag(const int* flags, int word)
 {
     return __hip_atomic_load(&flags[word], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-// The rebuild flag: the number of the first force pass that must not run on
-// the present lists, doubled, plus one (so that it is never 0).
-__host__ __device__ inline uint32_t rebuild_at(uint32_t pass) { return pass << 1 | 1u; }
-// Whether force pass `pass` has to wait for that rebuild.  A pass and the
-// drift that it ends with, which asks for the next one, never confuse each
-// other.
-__host__ __device__ inline bool waits_for_rebuild(uint32_t flag, uint32_t pass)
-{
-    return flag != 0 && (int32_t)(flag - rebuild_at(pass)) <= 0;
 }
 
 // What integrate() asks of the list upkeep, for the force pass `pass`.  One
@@ -3379,9 +3369,12 @@ int run_passes(dem_ctx* ctx, int64_t n, int erase, int last_kick, bool steps)
         if ((r = read_flags(ctx)) != 0) return r;
         // (a diverged state is never rebuilt: its passes count, and do nothing)
         const uint32_t flag = ctx->h_flags[F_NONFINITE] ? 0u : (uint32_t)ctx->h_flags[F_REBUILD];
-        int64_t idle = 0;  // launched passes that did nothing
-        if (flag) idle = std::max<int64_t>(0, (int32_t)(rebuild_at(ctx->passes) - flag) / 2 + 1);
-        idle = std::min(idle, sent - done);
+        // launched passes that did nothing: among those not yet counted, or a
+        // request was missed
+        const int64_t idle = flag ? idle_passes(flag, ctx->passes) : 0;
+        if (idle > sent - done)
+            return set_err(ctx, DEM_ERR_STATE, "internal error: " + std::to_string(idle) + " force passes waited for a "
+                                               "rebuild, of " + std::to_string(sent - done) + " in flight");
         for (int64_t k = 0; k < idle; ++k, --sent) unlaunch_force<NS>(ctx, sent < n ? KICK_BOTH : last_kick);
         if ((r = finish(sent)) != 0) return r;
         flying = 0;
