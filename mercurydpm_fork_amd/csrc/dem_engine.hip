@@ -3483,6 +3483,7 @@ int run_download(dem_ctx* ctx, double* const dst[6])
 {
     Dev<NS>& d = dev<NS>(ctx);
     const size_t n = (size_t)ctx->n;
+    if (std::none_of(dst, dst + 6, [](const double* a) { return a != nullptr; })) return DEM_OK;
     const bool small = ctx->n <= kSmallState;
     if (small)
         if (const int r = ensure_stage(ctx)) return r;

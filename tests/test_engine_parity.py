@@ -1251,3 +1251,20 @@ def test_rebuilds_asked_for_in_almost_every_pass(every):
             assert (t.n_steps, t.time, t.n_rebuilds, t.n_contacts) == (s.n_steps, s.time, s.n_rebuilds, s.n_contacts)
     assert rebuilds[0] >= 40 // (every + 1) and rebuilds[1] < 30 and rebuilds[3] >= 100 // (every + 1)
     assert_contacts_equal(batched, single)
+
+
+@pytest.mark.parametrize("n", [1, 8192, 8193])
+def test_no_array_wanted(n):
+    """dem_download_particles without any output array and dem_set_kinematics
+    without any input array do nothing, on either side of the largest system
+    whose state goes through pinned memory."""
+    sc = S.chute_hvm(n_flow=9000, seed=6, l=24.4, depth=10.0)
+    sc = _subset(sc, np.arange(n))
+    e = dem.Engine()
+    S.apply(e, sc)
+    a = e.download()
+    e._check(e.lib.dem_download_particles(e.h, *[None] * 6))
+    e.set_kinematics()
+    b = e.download()
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
