@@ -38,7 +38,8 @@ int dem_mlp_forward(dem_mlp* mlp, int64_t n, const double* x, double* y);
  * gradient with respect to every parameter (grad may be NULL) */
 int dem_mlp_gradient(dem_mlp* mlp, int64_t n, const double* x, const double* target, double* grad, double* loss);
 /* `epochs` full-batch Adam steps (beta 0.9 / 0.999, eps 1e-8) at learning
- * rate lr; loss: the loss before the last step */
+ * rate lr; loss: the loss before the last step (no step: of the present
+ * parameters) */
 int dem_mlp_train(dem_mlp* mlp, int64_t n, const double* x, const double* target, int32_t epochs, double lr,
                   double* loss);
 
@@ -68,7 +69,8 @@ int dem_closure_forward(dem_closure* net, int64_t n, const float* x, float* y);
 int dem_closure_gradient(dem_closure* net, int64_t n, const float* x, const float* target, float* grad,
                          float* loss);
 /* `epochs` full-batch Adam steps (beta 0.9 / 0.999, eps 1e-8) at learning
- * rate lr; loss: the loss before the last step */
+ * rate lr; loss: the loss before the last step (no step: of the present
+ * parameters) */
 int dem_closure_train(dem_closure* net, int64_t n, const float* x, const float* target, int32_t epochs, float lr,
                       float* loss);
 

@@ -764,6 +764,7 @@ int dem_closure_train(dem_closure* c, int64_t n, const float* x, const float* ta
         const float c1 = 1.0f - std::pow(0.9f, (float)c->step), c2 = 1.0f - std::pow(0.999f, (float)c->step);
         backward(c, (int)n, lr, c1, c2);
     }
+    if (epochs == 0 && loss) backward(c, (int)n, 0.0f, 1.0f, 1.0f);
     CCHK(hipGetLastError());
     if (loss) CCHK(hipMemcpyAsync(loss, c->loss, sizeof(float), hipMemcpyDeviceToHost, c->stream));
     CCHK(hipStreamSynchronize(c->stream));

@@ -330,6 +330,7 @@ int dem_mlp_train(dem_mlp* c, int64_t n, const double* x, const double* target, 
         hipLaunchKernelGGL(k_mlp_adam, dim3(blocks(kP)), dim3(kBlock), 0, c->stream, c->p, (const double*)c->g,
                            c->m, c->v, lr, 0.9, 0.999, 1e-8, ++c->adam_step);
     }
+    if (epochs == 0 && loss) launch_gradient(c, n);
     if (hipGetLastError() != hipSuccess) return DEM_ERR_DEVICE;
     if (loss && hipMemcpyAsync(loss, c->loss, sizeof(double), hipMemcpyDeviceToHost, c->stream) != hipSuccess)
         return DEM_ERR_DEVICE;

@@ -279,3 +279,22 @@ def test_closure128_on_held_out_angle_and_friction():
     print(f"held-out friction 0.45: mu_eff error per state {err_net:.4g} against the constant closure's "
           f"{err_const:.4g}")
     assert err_net < 0.5 * err_const, (err_net, err_const)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("net_of", [closure.MLP, closure.Closure], ids=["fp64", "bf16"])
+def test_no_epochs_returns_the_present_loss(net_of):
+    """Training for no epochs leaves the parameters and the Adam state alone
+    and returns the loss of the samples it was given, on a new network and
+    after training on other samples."""
+    x, t = samples(300, 8)
+    net, other = net_of(seed=4), net_of(seed=4)
+    assert net.train(x, t, 0) == net.gradient(x, t)[0] > 0.0
+    for k in (net, other):
+        k.train(x, 3.0 * t, 2)
+    p = net.params()
+    assert net.train(x, t, 0) == net.gradient(x, t)[0] != net.gradient(x, 3.0 * t)[0]
+    np.testing.assert_array_equal(net.params(), p)
+    for k in (net, other):
+        k.train(x, t, 2)
+    np.testing.assert_array_equal(net.params(), other.params())
