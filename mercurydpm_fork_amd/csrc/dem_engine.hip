@@ -1900,7 +1900,9 @@ constexpr double kSqrtPi = 1.7724538509055160272981674833411; // ExtendedMath.h:
 constexpr double kSqrt2 = 1.4142135623730950488016887242097;  // ExtendedMath.h:47
 constexpr int kCgFields = DEM_CG_FIELDS;
 
-constexpr int64_t kCgThreads = 2048 * 64;
+// see run_cg_z
+constexpr int64_t kCgMinThreads = 2048 * 64, kCgMaxThreads = 32768 * 64, kCgChunk = 256, kCgMaxChunk = 1024;
+constexpr size_t kCgKeep = 512u << 20;
 struct CgParams {
     int npts, chunk, nchunks, dims;
     double w, cutoff, prefactor;
@@ -2788,7 +2790,7 @@ struct dem_ctx {
     // pinned staging of the particle state of small systems (grow-only)
     double *h_stage = nullptr, *d_stage = nullptr;
     size_t stage_cap = 0;
-    // partial sums and output of dem_cg_z (grow-only, outlives re-uploads)
+    // partial sums and output of dem_cg_z (grows, kept up to kCgKeep bytes, outlives re-uploads)
     void* d_cg = nullptr;
     size_t cg_cap = 0;
     // index changes and lists of dem_remove_particles in place (grow-only)
@@ -3873,12 +3875,18 @@ int run_cg_z(dem_ctx* ctx, const dem_cg_config* cfg, double* out)
     c.volume = (cfg->max[0] - cfg->min[0]) * (cfg->max[1] - cfg->min[1]);
     c.stamp = (double)ctx->fc_pass;
     // One thread per point and chunk of particles: chunks of 4 particles or,
-    // where that would be more than 2048 wavefronts (and partial sums beyond
-    // 30 MB), more.  A thread's chunk is a serial chain, so few long ones leave
-    // the GPU idle: 105,000 spheres on 64 points took 1.76 ms with chunks of
-    // 1024 (103 wavefronts), 0.42, 0.27, 0.21, 0.23 and 0.27 ms with 512, 1024,
-    // 2048, 4096 and 8192 wavefronts.
-    c.chunk = (int)std::min<int64_t>(ctx->n, std::max<int64_t>(4, (ctx->n * c.npts + kCgThreads - 1) / kCgThreads));
+    // where that would be more than 2048 wavefronts, more; from chunks of 256 on
+    // more wavefronts, up to 32,768 (and 490 MB of partial sums), then chunks up
+    // to 1024.  A thread's chunk is a serial chain, so few long ones leave the
+    // GPU idle; many short ones write more partial sums.  ms with 2048, 4096,
+    // 8192, 16,384 and 32,768 wavefronts: 105,000 spheres on 64 points 0.20,
+    // 0.21, 0.25, 0.32, 0.59, on 1001 points 1.66, 1.31, 1.31, 1.31, 1.43; 2.08M
+    // spheres on 64 points 2.59, 2.40, 2.50, 2.65, 2.80, on 1001 points 32.7,
+    // 27.1, 24.5, 22.8, 21.4 (chunks of 1024 in every case: 1.5, 1.8, 4.1 and
+    // 22.5 ms); on 9001 points 161 with 32,768, 155 with chunks of 1024.
+    const int64_t work = ctx->n * c.npts;
+    const int64_t threads = std::max(kCgMinThreads, std::min(kCgMaxThreads, work / kCgChunk));
+    c.chunk = (int)std::min(ctx->n, std::min(kCgMaxChunk, std::max<int64_t>(4, (work + threads - 1) / threads)));
     c.nchunks = (int)std::max<int64_t>(1, (ctx->n + c.chunk - 1) / c.chunk);
     const size_t np = (size_t)c.nchunks * c.npts * kCgFields;
     const size_t bytes = sizeof(double) * (np + (size_t)c.npts * kCgFields);
@@ -3900,6 +3908,11 @@ int run_cg_z(dem_ctx* ctx, const dem_cg_config* cfg, double* out)
     if (e == hipSuccess)
         e = hipMemcpyAsync(out, dout, sizeof(double) * (size_t)c.npts * kCgFields, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (ctx->cg_cap > kCgKeep) {
+        (void)hipFree(ctx->d_cg);
+        ctx->d_cg = nullptr;
+        ctx->cg_cap = 0;
+    }
     if (e != hipSuccess) return set_err(ctx, DEM_ERR_DEVICE, std::string("dem_cg_z: ") + hipGetErrorString(e));
     return DEM_OK;
 }

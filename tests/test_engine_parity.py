@@ -8,6 +8,8 @@ per-particle sum of the magnitudes of the terms summed into them (the
 engine gathers a particle's contacts in list order, the reference in handler
 order, so only round-off of the sum may differ).
 """
+import math
+
 import numpy as np
 import pytest
 
@@ -1268,3 +1270,41 @@ def test_no_array_wanted(n):
     b = e.download()
     for k in a:
         np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+def test_cg_chunks_of_many_points():
+    """Particles and points (33.7 million together) for which a thread's
+    chunk has reached 257 particles, the last one shorter: the oracle's
+    fields, whose sums run over all particles in order, within rounding."""
+    sc = S.mixture(n=601, seed=94, lx=8.0, ly=8.0, lz=8.0, inflate=1.1, laws="hvm", periodic=(True, True),
+                   walls=("bottom",))
+    g, o = make_pair(sc)
+    for e in (g, o):
+        e.compute_forces()
+    a, b = (e.cg_z(56_003, 0.6, (0.0, 0.0, 0.0), (8.0, 8.0, 8.5)) for e in (g, o))
+    scale = np.abs(b).max(axis=0)
+    # (the bar of test_engine_cg_vs_oracle)
+    assert np.all(np.abs(a - b) <= 1e-10 * scale), np.max(np.abs(a - b) / np.maximum(scale, 1e-300))
+
+
+def test_cg_longest_chunks():
+    """Particles and points (3.0 billion together) for which chunks stay at
+    1024 particles and the partial sums are not kept: volume fraction, density
+    and momentum at a few points against the sums written out, and the same
+    bits from a second call."""
+    sc = S.chute_hvm(n_flow=100_000, seed=5, depth=20.0)
+    g = dem.Engine()
+    S.apply(g, sc)
+    g.compute_forces()
+    st, w, points = sc.state, 0.5, 30_011
+    lo, hi = float(st.x[:, 2].min()) - 1.0, float(st.x[:, 2].max()) + 1.0
+    a = g.cg_z(points, w, (0.0, 0.0, lo), (10.0, 20.0, hi))
+    np.testing.assert_array_equal(a, g.cg_z(points, w, (0.0, 0.0, lo), (10.0, 20.0, hi)))
+    free = st.inv_mass != 0.0
+    z, r, m, v = st.x[free, 2], st.radius[free], 1.0 / st.inv_mass[free], st.v[free]
+    for k in (0, 777, 15_005, 29_000, points - 1):
+        d2 = (z - (lo + (hi - lo) * (k + 0.5) / points)) ** 2
+        phi = np.where(d2 <= 9.0 * w * w, np.exp(-d2 / (2.0 * w * w)), 0.0)
+        phi /= np.sqrt(2.0 * np.pi) * w * math.erf(3.0 / np.sqrt(2.0)) * 10.0 * 20.0
+        want = [np.sum(4.0 / 3.0 * np.pi * r ** 3 * phi), np.sum(m * phi), *np.sum(v * (m * phi)[:, None], axis=0)]
+        np.testing.assert_allclose(a[k, :5], want, rtol=1e-10, atol=1e-10 * np.abs(a[:, :5]).max())
