@@ -170,9 +170,9 @@ struct Dev {
     // owner's own list << 8 | owner's lane << 14.
     uint2* nbrc;
     uint32_t* gtot;
-    // the entries of nbrc that can come into contact before the next pruning,
-    // in the same layout (k_force)
-    uint2* nbri;
+    // the wavefront's entries that can come into contact before the next
+    // pruning, itot[w] of them, follow its lists in the same region from the
+    // next multiple of 16 entries on, if they fit there (k_force)
     uint32_t* itot;
     // contact records
     Rec<NS>* rec[2];
@@ -1294,8 +1294,12 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 // list order; the passes that follow walk those (about 3 per particle), which
 // holds until some particle has moved half the smaller skin: integrate() then
 // asks the next pass to prune (a word for even and one for odd passes, with the
-// pass's number: a pass and the requests made in it never meet).  Every contact is found, in the same
-// order, so the results are bit-identical.
+// pass's number: a pass and the requests made in it never meet).  Every contact
+// is found, in the same order, so the results are bit-identical.  They lie behind
+// the whole lists in the wavefront's region, where lists that fill less than
+// about two thirds of max_neighbors leave room; fuller ones are walked whole
+// (an array of their own, the same times, took 512 B more per particle: 4% of
+// what a GPU holds).
 //
 // What bounds it (2M chute, 0.2 to 0.9 contacts per particle): the state alone,
 // read and written with the integration, takes 163 us (770 MB, 4.7 TB/s, the
@@ -1575,9 +1579,13 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     // entries starting at wbase * stride: the pruned ones, or all of them in a
     // pass that prunes
     const bool prune = prune_at == pass;
-    const uint2* __restrict__ list = prune ? d.nbrc : d.nbri;
-    const int total = __builtin_amdgcn_readfirstlane((int)(prune ? total_all : total_pruned));
-    const size_t lbase = (size_t)wbase * p.maxn;
+    const uint32_t pruned_at = (total_all + 15u) & ~15u;
+    const uint32_t room = (uint32_t)(p.group * p.maxn) - pruned_at;
+    const bool whole = prune || total_pruned > room;
+    const int total = __builtin_amdgcn_readfirstlane((int)(whole ? total_all : total_pruned));
+    const size_t region = (size_t)wbase * p.maxn;
+    const uint2* list = d.nbrc + region + (whole ? 0u : pruned_at);
+    uint2* pruned = d.nbrc + region + pruned_at;
     uint32_t kept = 0;
     unsigned long long touched = 0;
     V3 F = zero3(), T = zero3();
@@ -1590,7 +1598,7 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
 #pragma unroll
         for (int u = 0; u < kScanU; ++u) {
             const int e = e0 + 64 * u + lane;
-            en[u] = e < total ? list[lbase + (size_t)e] : make_uint2(0u, 0u);
+            en[u] = e < total ? list[e] : make_uint2(0u, 0u);
         }
 #pragma unroll
         for (int u = 0; u < kScanU; ++u)
@@ -1634,8 +1642,9 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
             }
             if (prune) {
                 const unsigned long long nb = __ballot(near);
-                if (near) d.nbri[lbase + kept + lane_prefix(nb)] = en[u];
-                kept += (uint32_t)__popcll(nb);
+                const uint32_t upto = kept + (uint32_t)__popcll(nb);
+                if (near && upto <= room) pruned[kept + lane_prefix(nb)] = en[u];
+                kept = upto;
             }
             const unsigned long long ballot = __ballot(contact);
             if (contact) L.q[qn + lane_prefix(ballot)] = entry;
@@ -2943,7 +2952,7 @@ int alloc_particles(dem_ctx* ctx, int64_t n)
     A(d.t_id, n) A(d.t_orig, n) A(d.t_spc, n) A(d.t_cellc, n);
     const size_t slots = (size_t)n * ctx->maxn_cfg;
     const size_t wslots_packed = ((size_t)n + 63) / 64 * 64 * ctx->maxn_cfg;
-    A(d.nbr, slots) A(d.ncount, n) A(d.nbrc, wslots_packed) A(d.nbri, wslots_packed);
+    A(d.nbr, slots) A(d.ncount, n) A(d.nbrc, wslots_packed);
     const size_t waves = ((size_t)n + ctx->prm.group - 1) / ctx->prm.group;
     A(d.gtot, waves) A(d.itot, waves);
     A(d.rec[0], slots) A(d.rec[1], slots) A(d.mask[0], n) A(d.mask[1], n) A(d.fc, slots) A(d.ftc, slots);

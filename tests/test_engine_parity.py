@@ -1308,3 +1308,28 @@ def test_cg_longest_chunks():
         phi /= np.sqrt(2.0 * np.pi) * w * math.erf(3.0 / np.sqrt(2.0)) * 10.0 * 20.0
         want = [np.sum(4.0 / 3.0 * np.pi * r ** 3 * phi), np.sum(m * phi), *np.sum(v * (m * phi)[:, None], axis=0)]
         np.testing.assert_allclose(a[k, :5], want, rtol=1e-10, atol=1e-10 * np.abs(a[:, :5]).max())
+
+
+@pytest.mark.parametrize("most", [6, 7, 8, 9, 12, 64])
+def test_pruned_lists_that_do_not_fit(most):
+    """A wavefront's pruned lists lie behind its lists in what max_neighbors
+    leaves free, or its whole lists are walked: a jittered lattice with six
+    neighbours each, about half of them within the pruned lists' skin, in
+    room for 0 to 58 more.  The contacts of the oracle, step by step."""
+    m = 6
+    rng = np.random.default_rng(7)
+    x = np.stack(np.meshgrid(*[np.arange(m) + 0.5] * 3, indexing="ij"), -1).reshape(-1, 3)
+    x = x + rng.uniform(-0.02, 0.02, x.shape) + np.where(np.arange(len(x)) % 3 == 0, 0.03, 0.0)[:, None]
+    sp = S.hertz_mindlin_species(tc=0.01)
+    st = S.make_state(x, rng.normal(0.0, 0.3, x.shape), np.full(len(x), 0.5), np.zeros(len(x), np.int32), [sp])
+    sc = S.Scenario("lattice", [sp], [], [S.periodic_boundary(a, 0.0, float(m)) for a in range(3)], (0.0, 0.0, 0.0),
+                    sp.info_tc / 50, st)
+    g, o = make_pair(sc, skin=0.15, max_neighbors=most)
+    for e in (g, o):
+        e.compute_forces()
+    assert assert_contacts_equal(g, o) > 50
+    for _ in range(4):
+        for e in (g, o):
+            e.step(4)
+        assert_contacts_close(g, o)
+    assert g.stats().n_rebuilds == 1
