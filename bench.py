@@ -23,9 +23,11 @@ step; HIP-event timed on the engine's stream) with the whole-step byte model
 host's cores, on a bounded sample of the same state).
 """
 import argparse
+import hashlib
 import json
 import math
 import os
+import re
 import sys
 import time
 
@@ -39,19 +41,40 @@ HBM_PEAK_GBS = 8000.0
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "k_force_chute2M_traffic.md")
 
 
-def measured_traffic():
-    """(traffic_bytes_per_launch, contacts_per_particle of the profiled state)
-    from the committed counter summary, or (None, None)."""
-    traffic, cbar = None, None
+# what the compiled force kernel depends on
+ENGINE_SOURCES = ("mercurydpm_fork_amd/csrc/dem_engine.hip", "mercurydpm_fork_amd/csrc/dem_laws.h",
+                  "mercurydpm_fork_amd/csrc/dem_laws_mixed.h", "mercurydpm_fork_amd/csrc/dem_passes.h",
+                  "mercurydpm_fork_amd/csrc/dem_vec.h", "mercurydpm_fork_amd/csrc/dem_walls.h",
+                  "include/mercurydpm_dem.h")
+
+
+def engine_source_hash():
+    """Of the engine's sources without comments and white space: names the
+    build that a profile was taken of."""
+    h = hashlib.sha256()
+    for name in ENGINE_SOURCES:
+        with open(os.path.join(ROOT, name)) as f:
+            text = re.sub(r"/\*.*?\*/|//[^\n]*", "", f.read(), flags=re.S)
+        h.update(re.sub(r"\s+", "", text).encode())
+    return h.hexdigest()[:16]
+
+
+def traffic_profile():
+    """The figures of the committed counter summary: traffic_bytes_per_launch,
+    contacts_per_particle, pruned_entries_per_particle, passes_per_pruning (as
+    floats) and engine_source_hash, of the state that it was taken on."""
+    out = {}
     try:
         for line in open(TRAFFIC_PROFILE):
-            if line.startswith("traffic_bytes_per_launch:"):
-                traffic = int(line.split(":", 1)[1])
-            if line.startswith("contacts_per_particle:"):
-                cbar = float(line.split(":", 1)[1])
+            key, sep, val = line.partition(":")
+            if sep and key in ("traffic_bytes_per_launch", "contacts_per_particle", "pruned_entries_per_particle",
+                               "passes_per_pruning"):
+                out[key] = float(val)
+            elif sep and key == "engine_source_hash":
+                out[key] = val.strip()
     except OSError:
         pass
-    return traffic, cbar
+    return out
 
 
 def parse():
@@ -297,13 +320,21 @@ def b_alg(cbar, mixed=False):
     return (216.0 if mixed else 264.0) + 64.0 * cbar
 
 
-def fused_bytes(cbar, lbar):
+def fused_bytes(cbar, walked):
     """The force kernel's own model (it also integrates): own state in
-    (posr, vel, omg, quat, disp: 160; mask, list length, species, wall mask:
-    20) and out (posr, vel, omg, quat, disp: 160; masks: 12), 8 B per list
-    entry (partner index and reverse slot, one 8-byte load), 64 B per pair in
-    contact."""
-    return 352.0 + 8.0 * lbar + 64.0 * cbar
+    (posr, vel, omg, quat, disp: 160; mask, species, wall mask: 16) and out
+    (posr, vel, omg, quat, disp: 160; masks: 12), 8 B per list entry walked,
+    64 B per pair in contact."""
+    return 348.0 + 8.0 * walked + 64.0 * cbar
+
+
+def entries_walked(lbar, prof):
+    """List entries that a force pass reads or writes per particle, on average:
+    the pruned lists, and in a pass that prunes the whole lists as well (None
+    without the profile's figures)."""
+    if "pruned_entries_per_particle" not in prof or not prof.get("passes_per_pruning"):
+        return None
+    return prof["pruned_entries_per_particle"] + lbar / prof["passes_per_pruning"]
 
 
 def cpu_threads():
@@ -463,7 +494,9 @@ def main():
     mixed_run = a.precision == "mixed"
     balg = b_alg(cbar, mixed_run)
     achieved = balg * n_total / (force_ms * 1e-3) / 1e9
-    bfused = fused_bytes(cbar, lbar)
+    prof = traffic_profile()
+    walked = entries_walked(lbar, prof)
+    bfused = None if walked is None else fused_bytes(cbar, walked)
     log(f"timed {a.steps} steps in {elapsed:.3f}s: force+integration {force_ms:.3f} ms, kick "
         f"{st.t_kick_ms / max(st.n_timed_steps, 1):.3f} ms, rebuild "
         f"{st.t_rebuild_ms / max(st.n_timed_steps, 1):.3f} ms per step; {st.n_rebuilds - rb0} rebuilds in the "
@@ -521,7 +554,9 @@ def main():
         o.close()
         log(f"cpu baseline: {cpu['value']:.3g} particle-steps/s on {got} threads ({cpu['seconds']} s)")
 
-    traffic, traffic_cbar = measured_traffic()
+    # (counted on one build: another one's traffic is not known)
+    traffic_current = not a.engine_lib and prof.get("engine_source_hash") == engine_source_hash()
+    traffic = int(prof["traffic_bytes_per_launch"]) if traffic_current and "traffic_bytes_per_launch" in prof else None
     out = {
         "metric": "particle-steps/sec at 2M polydisperse spheres",
         "value": value,
@@ -549,17 +584,21 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 5),
                      "traffic": traffic if a.n == 2_000_000 else None,
-                     "traffic_contacts_per_particle": traffic_cbar,
+                     "traffic_contacts_per_particle": prof.get("contacts_per_particle"),
                      "traffic_source": "profiles/k_force_chute2M_traffic.md (rocprofv3 FETCH_SIZE, WRITE_SIZE, "
-                                       "copy-calibrated)",
+                                       "copy-calibrated)" +
+                                       ("" if traffic_current else "; of another build than this one: not reported"),
                      "kernel": "k_force", "kernel_ms": round(force_ms, 4),
                      "bytes_per_particle": round(balg, 2),
                      "bytes_model": "264 + 64 C (whole step, per particle of the launch)",
                      "particles_per_launch": n_total,
-                     "fused_kernel_model": {"bytes_per_particle": round(bfused, 2),
-                                            "achieved": round(bfused * n_total / (force_ms * 1e-3) / 1e9, 2),
-                                            "frac": round(bfused * n_total / (force_ms * 1e-3) / 1e9 /
-                                                          HBM_PEAK_GBS, 5)}},
+                     "fused_kernel_model": None if bfused is None else {
+                         "bytes_per_particle": round(bfused, 2),
+                         "list_entries_walked_per_particle": round(walked, 3),
+                         "list_entries_source": "profiles/k_force_chute2M_traffic.md (pruned entries and passes per "
+                                                "pruning, counted on the state after the default run)",
+                         "achieved": round(bfused * n_total / (force_ms * 1e-3) / 1e9, 2),
+                         "frac": round(bfused * n_total / (force_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 5)}},
         "run_average": run_avg,
         "steady_window": steady,
         "cpu_baseline": cpu,

@@ -8,8 +8,9 @@
 // gradient (dW = dZ^T H).  One kernel takes a tile of samples through the whole
 // network: inference keeps everything between the input and the output in
 // registers and LDS, training also goes back through the network and adds the
-// tile's gradient, and a second kernel sums the blocks' gradients in block
-// order (so they are the same bits on every run) and applies Adam.  The 4-wide
+// tile's gradient, and a second kernel sums the blocks' gradients in a fixed
+// order (four runs of blocks, then the runs: the same bits every time) and
+// applies Adam.  The 4-wide
 // input layer and the 2-wide output layer are too narrow for a tile and run on
 // the vector units with the same BF16 weights.  Activations fed to a matrix
 // instruction are rounded to BF16 (round to nearest even); pre-activations,

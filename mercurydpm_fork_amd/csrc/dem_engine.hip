@@ -54,8 +54,9 @@ constexpr int kMaxSlabs = 64;
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64; // wavefronts per block
 // Skin of the pruned lists, as a fraction of the Verlet skin: a smaller one
-// keeps fewer entries and prunes more often.  2M chute, us per force pass at
-// 0.08, 0.14, 0.2, 0.3, 0.45: 447, 443, 444, 450, 457 (462 without pruning).
+// keeps fewer entries and prunes more often.  A thin bed of 2.08M spheres (0.2 to
+// 0.9 contacts per particle), us per force pass at 0.08, 0.14, 0.2, 0.3, 0.45:
+// 447, 443, 444, 450, 457 (462 without pruning).
 constexpr double kInnerSkin = 0.2;
 // Particles up to which a wavefront of the force kernel takes 16 and 32
 // particles instead of 64.  A wavefront's pass is a chain of dependent loads
@@ -898,9 +899,9 @@ struct ListLds {
 // The per-particle sweep need not read the candidates' cells where a sweep
 // cannot meet a bucket twice: every bucket of a level is then met for one cell,
 // and a particle of another cell that shares the bucket is far away, so that
-// the distance test drops it (211,000 spheres: 315 us per build, 2.08M: 2.2 ms; 388 us and 3.15 ms with the
-// cell test and in one kernel with the wavefront sweep, whose LDS and registers
-// it does not need).
+// the distance test drops it (211,000 spheres: 315 us per build, 2.08M: 2.2 ms;
+// 388 us and 3.15 ms with the cell test and in one kernel with the wavefront
+// sweep, whose LDS and registers it does not need).
 template <int NS>
 __device__ inline void sweep_cells(Dev<NS>& d, const Params& p, int m, const int lo[3], const int hi[3], const int nc[3],
                                    int i, V3 xi, double ri, uint32_t idi, bool fixed_i, int& cnt)
@@ -1282,18 +1283,19 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 // history record.
 // A packed list entry names its owner and its slot in the owner's list: finding
 // them by a binary search over the owners' list lengths in LDS cost six
-// dependent LDS reads per entry (2M chute, 600 steps and the state read back:
+// dependent LDS reads per entry (2.08M spheres, 600 steps and the state read back:
 // 423 ms with the search and both half-kicks' increments computed apart, 413
 // without).
 //
-// Pruned lists.  Of a Verlet list's 7.3 entries per particle on the chute about
-// 2 are in contact; most of the rest cannot come into contact for many steps,
-// but each cost a list entry, a 32-byte gather of the partner's position and a
-// test in every step.  A pass that prunes walks the whole lists and keeps the
-// entries within the sum of the radii plus a smaller skin (Params::inner), in
-// list order; the passes that follow walk those (about 3 per particle), which
-// holds until some particle has moved half the smaller skin: integrate() then
-// asks the next pass to prune (a word for even and one for odd passes, with the
+// Pruned lists.  Of a Verlet list's 7.4 entries per particle on the developed
+// chute 2.7 are in contact; of the rest many cannot come into contact for many
+// steps, but each cost a list entry, a 32-byte gather of the partner's position
+// and a test in every step.  A pass that prunes walks the whole lists and keeps
+// the entries within the sum of the radii plus a smaller skin (Params::inner), in
+// list order; the passes that follow walk those (5.5 per particle on the
+// developed chute, where one pass in 30 prunes; about 3 on the thin bed below),
+// which holds until some particle has moved half the smaller skin: integrate()
+// then asks the next pass to prune (a word for even and one for odd passes, with the
 // pass's number: a pass and the requests made in it never meet).  Every contact
 // is found, in the same order, so the results are bit-identical.  They lie behind
 // the whole lists in the wavefront's region, where lists that fill less than
@@ -1301,13 +1303,15 @@ __device__ inline void wall_geometry(V3 x, double r, double distance, V3 n, Cont
 // (an array of their own, the same times, took 512 B more per particle: 4% of
 // what a GPU holds).
 //
-// What bounds it (2M chute, 0.2 to 0.9 contacts per particle): the state alone,
-// read and written with the integration, takes 163 us (770 MB, 4.7 TB/s, the
-// rate of a large copy); walking the pruned lists adds about 80 us and the
-// contacts 70 to 190, waiting for gathers.  437 us per pass with pruning and
-// with the sums taken lane to lane (16 KB less LDS per block), 462 before; 424
-// since a pass loads all it starts from at once.  Four wavefronts per SIMD (128 registers, spilling) took 491, two lanes
-// loading each record together 441.
+// What bounds it: waiting for gathers.  2.08M spheres of a thin bed (0.2 to 0.9
+// contacts per particle): the state alone, read and written with the
+// integration, takes 163 us (770 MB, 4.7 TB/s, the rate of a large copy);
+// walking the pruned lists adds about 80 us and the contacts 70 to 190.  437 us
+// per pass with pruning and with the sums taken lane to lane (16 KB less LDS per
+// block), 462 before; 424 since a pass loads all it starts from at once.  Four
+// wavefronts per SIMD (128 registers, spilling) took 491, two lanes loading each
+// record together 441.  The developed chute of the same size (1.36 contacts per
+// particle, 5.5 pruned entries): 498 us per pass, 535 before the pruned lists.
 
 // v of lane src
 __device__ inline V3 wave_get(V3 v, int src)
@@ -1529,7 +1533,7 @@ __global__ void __launch_bounds__(kBlock) FORCE_WAVES_ATTR k_force(Dev<NS> d, Pa
     // Everything that the pass starts from is loaded at once: the flag words,
     // the owners' state and the lengths of both packed lists.  (The flags change
     // during the pass only in ways it must not see, or need not: a cached load
-    // will do.  2M chute: 436 us per pass with the flags read one after another
+    // will do.  2.08M spheres: 436 us per pass with the flags read one after another
     // past the caches and the rest after them, 424 so.)
     const int nonfinite = load_flag(d.flags, F_NONFINITE);
     const uint32_t rebuild = (uint32_t)load_flag(d.flags, F_REBUILD);
@@ -3096,7 +3100,7 @@ void launch_kick(dem_ctx* ctx, int after, int before)
 int read_flags(dem_ctx* ctx)
 {
     int* f = ctx->h_flags;
-    // (a kernel that writes 16 words to pinned memory is quicker than a copy)
+    // (a kernel that writes the words to pinned memory is quicker than a copy)
     hipLaunchKernelGGL(k_flags_to_host, dim3(1), dim3(64), 0, ctx->stream, (const int*)ctx->d_flags, f);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
