@@ -386,7 +386,9 @@ __device__ inline int load_flag(const int* flags, int word)
 // request yet: particles that move together cross the skin in the same pass,
 // and their stores to the one word wait for each other (2.0M spheres of one
 // speed, no contacts: a pass after which none asks takes 0.137 ms; one after
-// which all ask took 1.31 ms with a store per lane, and takes 0.18 ms so).
+// which all ask took 1.31 ms with a store per lane, and takes 0.18 ms so.  It is
+// the look at the word that does it: one store per wavefront without it is as
+// slow as one per lane).
 enum { NEEDS_REBUILD = 1, NEEDS_PRUNE = 2 };
 __device__ inline bool write_request(int* word, int value)
 {
